@@ -18,7 +18,7 @@ CSRC = HERE / "csrc"
 BUILD = HERE / "_build"
 LIB = HERE / "libneon_hip.so"
 
-SOURCES = ["engine.hip", "newton.hip", "eigen.hip", "capi.hip", "meshgen.cpp", "loads.cpp"]
+SOURCES = ["engine.hip", "grid_krylov.hip", "newton.hip", "eigen.hip", "capi.hip", "meshgen.cpp", "loads.cpp"]
 # the measurement library (include/neon_hip_measure.h): timing probes linked against LIB
 MEASURE_SOURCES = ["measure.hip"]
 MEASURE_LIB = HERE / "libneon_hip_measure.so"

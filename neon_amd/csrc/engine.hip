@@ -229,10 +229,11 @@ krylov_engine::krylov_engine(hipStream_t s) : s_(s)
 {
     // partials, then their total (totals_kernel)
     for (auto& p : part_) p.resize(kMaxPartials + 1);
-    state_.resize(2);
+    // two ping-ponged states; the resident grids' state and their abort word
+    state_.resize(4);
     scalar_.resize(1);
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_state_), sizeof(krylov_state)));
-    NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ring_), 2 * sizeof(krylov_state)));
+    NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ring_), 4 * sizeof(krylov_state)));
     for (auto& e : ring_events_) NEON_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_scalar_), sizeof(double)));
 }
@@ -288,9 +289,7 @@ void krylov_engine::jacobi64(const linear_operator& A, double* minv, int eigen_r
     NEON_CHECK_HIP(hipGetLastError());
 }
 
-namespace
-{
-solve_result finish(const krylov_state& s, int criterion)
+solve_result finish_solve(const krylov_state& s, int criterion)
 {
     solve_result r;
     r.iterations = s.it;
@@ -305,7 +304,6 @@ solve_result finish(const krylov_state& s, int criterion)
     }
     return r;
 }
-} // namespace
 
 // Drives a device-resident Krylov loop: `batch` launches poll_every iterations (advancing
 // `launched`; the state after `launched` iterations is st[launched & 1]).  The host keeps one
@@ -339,7 +337,6 @@ void krylov_engine::run_batches(krylov_state* st, int64_t& launched, Batch&& bat
     NEON_CHECK_HIP(hipMemcpyAsync(host_state_, st + (launched & 1), sizeof(krylov_state), hipMemcpyDeviceToHost, s_));
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
 }
-
 // Jacobi-PCG in FP64.  Per iteration: SpMV fused with the block partials of p.Ap, their total
 // (one block: the SpMV has one partial per slice quadruple, which every update block would
 // otherwise reduce), the r update fused with the partials of r.r and r.z, and the x and p
@@ -351,6 +348,8 @@ void krylov_engine::run_batches(krylov_state* st, int64_t& launched, Batch&& bat
 solve_result krylov_engine::cg64(const linear_operator& A, const double* b, double* x, const double* minv,
                                  int criterion, double tol, int32_t max_it, const krylov_work* work)
 {
+    solve_result res;
+    if (cg64_grid(A, b, x, minv, criterion, tol, max_it, work, res)) return res;
     int64_t const n = A.n;
     double *r = nullptr, *p = nullptr, *Ap = nullptr;
     if (work)
@@ -373,7 +372,6 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
     cg_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, criterion, tol, max_it);
     NEON_CHECK_HIP(hipGetLastError());
 
-    solve_result res;
     int64_t launched = 0;
     run_batches(st, launched, [&] {
         for (int k = 0; k < poll_every; ++k, ++launched)
@@ -389,7 +387,7 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
                                                        criterion, tol, max_it);
         }
     });
-    res = finish(*host_state_, criterion);
+    res = finish_solve(*host_state_, criterion);
     // SpMV launches that did work: Eigen's rule counts the converging iteration's SpMV
     // outside `iterations`; the CUDA rule counts every iteration.
     res.spmv = std::min<int64_t>(
@@ -659,7 +657,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     mixed_fold_kernel<<<nb, kBlock, 0, s_>>>(n, x, x32, p32, part_pAp, st + (launched & 1), 1, minv64_scaled);
     NEON_CHECK_HIP(hipGetLastError());
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
-    solve_result res = finish(*host_state_, NEON_STOP_RELATIVE);
+    solve_result res = finish_solve(*host_state_, NEON_STOP_RELATIVE);
     res.refinements = host_state_->restarts;
     int64_t const inner = res.iterations + (host_state_->done == KRYLOV_CONVERGED ? 1 : 0);
     res.spmv = inner + res.refinements;
@@ -676,6 +674,12 @@ __global__ __launch_bounds__(kBlock) void fill_kernel(int64_t n, T v, T* __restr
     if (i < n) x[i] = v;
 }
 } // namespace
+
+void fill_zero(hipStream_t s, int64_t n, double* x)
+{
+    fill_kernel<double><<<grid_for(n), kBlock, 0, s>>>(n, 0.0, x);
+    NEON_CHECK_HIP(hipGetLastError());
+}
 
 void fill_ones(hipStream_t s, int64_t n, double* x)
 {
@@ -1710,6 +1714,8 @@ void device_mesh::attach_sliced(linear_operator& A, int precision, bool index32)
     A.sell = true;
     A.sym = false;
     A.slices = slices_;
+    A.sell_steps = max_degree_;
+    A.sell_mean = double(sell_steps_) / slices_;
     A.sptr = sptr_.data();
     A.snode = snode_.data();
     A.slane = slane_.data();
@@ -1865,6 +1871,7 @@ void device_mesh::build_symmetric_pattern()
     sym_slots_ = int32_t(sched.size());
     sym_records_ = records;
     sym_max_entries_ = max_entries;
+    sym_mean_entries_ = double(eptr[slices_]) / slices_;
     sym_ok_ = true;
 }
 
@@ -1943,6 +1950,8 @@ void device_mesh::attach_symmetric(linear_operator& A, int precision, const doub
     A.slices = slices_;
     A.sym_slots = sym_slots_;
     A.sym_records = sym_records_;
+    A.sym_entries = sym_max_entries_;
+    A.sym_mean = sym_mean_entries_;
     A.sym_sched = sym_sched_.data();
     A.sym_rdiag = sym_rdiag_.data();
     A.sym_eptr = sym_eptr_.data();

@@ -40,6 +40,11 @@ public:
         }
         count = n;
     }
+    // at least n entries (the contents are lost when it grows)
+    void reserve(size_t n)
+    {
+        if (n > count) resize(n);
+    }
     void release()
     {
         if (ptr) (void)hipFree(ptr);
@@ -119,6 +124,8 @@ struct linear_operator
     // sliced copy of the node-block values (sell_matrix layout); the SpMV uses it when set
     bool sell = false;
     int32_t slices = 0;
+    int32_t sell_steps = 0; // largest and mean number of steps of a slice
+    double sell_mean = 0.0;
     const int32_t* sptr = nullptr;
     const int32_t* snode = nullptr;
     const int32_t* slane = nullptr;
@@ -133,6 +140,8 @@ struct linear_operator
     bool sym = false;
     int32_t sym_slots = 0;
     int64_t sym_records = 0;
+    int32_t sym_entries = 0; // largest and mean number of entries of a slice
+    double sym_mean = 0.0;
     const int32_t* sym_sched = nullptr;
     const int32_t* sym_rdiag = nullptr;
     const int32_t* sym_eptr = nullptr;
@@ -158,7 +167,16 @@ struct krylov_work
 {
     double *r = nullptr, *p = nullptr, *Ap = nullptr;
     double *r0 = nullptr, *v = nullptr, *s = nullptr, *t = nullptr, *p_hat = nullptr, *s_hat = nullptr;
+    // the resident-grid loops' vectors instead: ring_size doubles, none of the above but r among them
+    double* ring = nullptr;
+    int64_t ring_size = 0;
 };
+
+struct grid_link; // grid_kernels.hpp
+// Doubles of the ring that a resident grid's iterations publish their vectors to (64 MiB; at
+// least 8 iterations' worth)
+constexpr int64_t kGridRing = int64_t(1) << 23;
+solve_result finish_solve(const krylov_state& s, int criterion);
 
 class krylov_engine
 {
@@ -195,6 +213,9 @@ public:
     kernel_profiler* prof = nullptr;
     // iterations between convergence polls from the host
     int poll_every = 16;
+    // ticks (100 MHz) that a resident grid's workgroups wait for each other before the solve falls
+    // back to launches: another process may hold the compute units that some of them need
+    uint64_t grid_patience = 100ull * 1000 * 1000;
     // reliable-update trigger of the mixed-precision CG: ||r32|| < delta ||r at last update||
 #ifndef NEON_RELIABLE_DELTA
 #define NEON_RELIABLE_DELTA 0.1
@@ -218,11 +239,25 @@ private:
     device_array<double> part_[6];
     device_array<krylov_state> state_;
     krylov_state* host_state_ = nullptr;
-    // poll-ahead ring of run_batches: two pinned state snapshots and their events
+    // poll-ahead ring of run_batches and grid_run: two pinned state snapshots (of two states each
+    // for grid_run) and their events
     krylov_state* host_ring_ = nullptr;
     hipEvent_t ring_events_[2] = {nullptr, nullptr};
     template <typename Batch>
     void run_batches(krylov_state* st, int64_t& launched, Batch&& batch);
+    // resident-grid loops (grid_krylov.hip): false when the solve does not qualify or its grid
+    // gave up; the launch-per-phase loop then solves
+    bool cg64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion, double tol,
+                   int32_t max_it, const krylov_work* work, solve_result& out);
+    void grid_begin();
+    void grid_clear();
+    grid_link grid_next(uint32_t exchanges);
+    template <typename Batch>
+    bool grid_run(Batch&& batch);
+    int grid_device_ = 0, grid_units_ = 0;
+    uint32_t grid_epoch_ = 1;
+    device_array<uint64_t> grid_slots_;
+    device_array<double> grid_ring_, grid_r_;
     double* host_scalar_ = nullptr;
     device_array<double> scalar_;
     int64_t n_ = 0, n_mixed_ = 0;
@@ -391,6 +426,7 @@ private:
     // symmetric sliced layout: per-slice entries, records, the wave-slot schedule and the copies
     bool sym_ok_ = false;
     int32_t sym_slots_ = 0, sym_max_entries_ = 0;
+    double sym_mean_entries_ = 0.0;
     int64_t sym_records_ = 0;
     device_array<int32_t> sym_sched_, sym_rdiag_, sym_eptr_, sym_ent_, sym_rslice_, sym_roff_;
     mutable device_array<double> y64_;
@@ -412,6 +448,7 @@ private:
 
 void upload_hex8_tables();
 void convert_to_float(hipStream_t s, int64_t n, const double* x, float* y);
+void fill_zero(hipStream_t s, int64_t n, double* x);
 void fill_ones(hipStream_t s, int64_t n, double* x);
 void fill_ones(hipStream_t s, int64_t n, float* x);
 } // namespace neon_amd

@@ -1,0 +1,285 @@
+// Host side of the resident-grid Krylov loops (grid_kernels.hpp): which solves take them, the
+// shape of their grids, and the compute units they hold.
+#include "engine.hpp"
+#include "grid_kernels.hpp"
+
+#include <algorithm>
+#include <condition_variable>
+#include <mutex>
+
+namespace neon_amd
+{
+namespace
+{
+constexpr int64_t kGridLds = 160 * 1024 - 1024; // LDS of a compute unit less the static arrays
+
+// Compute units of each GPU that this process's resident grids may still take.  A grid's
+// workgroups wait for each other, so two grids that together exceed the GPU must not be in flight at
+// once; a solve waits here until the ones before it have left enough room.
+class unit_pool
+{
+public:
+    static unit_pool& of(int device)
+    {
+        static unit_pool pools[kDevices];
+        return pools[device];
+    }
+    static constexpr int kDevices = 64;
+    void take(int want, int units)
+    {
+        std::unique_lock<std::mutex> lock(m_);
+        cv_.wait(lock, [&] { return used_ + want <= units; });
+        used_ += want;
+    }
+    void give(int count)
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            used_ -= count;
+        }
+        cv_.notify_all();
+    }
+
+private:
+    std::mutex m_;
+    std::condition_variable cv_;
+    int used_ = 0;
+};
+
+class unit_hold
+{
+public:
+    unit_hold(int device, int want, int units) : pool_(unit_pool::of(device)), count_(want) { pool_.take(want, units); }
+    ~unit_hold() { pool_.give(count_); }
+    unit_hold(unit_hold const&) = delete;
+    unit_hold& operator=(unit_hold const&) = delete;
+
+private:
+    unit_pool& pool_;
+    int count_;
+};
+
+// LDS residency: `most` 8-byte vectors of the block's rows if they fit, else `least` of them
+bool fit_lds(grid_shape& g, int64_t extra, int most, int most_elems, int least, int least_elems)
+{
+    for (bool all : {true, false})
+    {
+        int64_t const bytes = int64_t(g.rows) * 8 * (all ? most : least) + extra;
+        if (bytes > kGridLds || g.rows > kGridThreads * (all ? most_elems : least_elems)) continue;
+        g.all = all;
+        g.lds = bytes;
+        return true;
+    }
+    return false;
+}
+
+// Shape of a sliced layout's grid: per_xcd slices on each XCD's list with `mean` records or entries
+// per slice, at most `most_items`.  Its cost is counted in items that a wavefront takes in turn, two
+// more for each round (a slice's head and the sums of its shares); a wavefront that has a slice to
+// itself waits for the longest slice.  Sharing a slice among wavefronts spreads few slices over all
+// compute units and evens out slices of unequal length; without need it only adds rounds (41 x 40 x
+// 38 cells, 1,050 slices: 14.4 us per product with one wavefront per slice, 15.1 with eight).
+bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_t most_items, int units)
+{
+    int const most = std::min(units, kGridMaxBlocks) / 8; // blocks per XCD
+    if (most < 1 || per_xcd < 1) return false;
+    double best = 0.0;
+    for (int wps : {1, 4, 8})
+    {
+        grid_shape t;
+        int const groups = kGridWaves / wps;
+        t.n = n;
+        t.wps = wps;
+        t.rounds = (per_xcd + groups * most - 1) / (groups * most);
+        if (wps == 4 && t.rounds > 1) continue;
+        t.per_xcd = std::min(most, (per_xcd + groups - 1) / groups);
+        t.blocks = 8 * t.per_xcd;
+        t.rows = t.rounds * groups * 192;
+        double const cost = t.rounds * (2.0 + (wps == 1 ? most_items : mean / wps));
+        int64_t const extra = (wps > 1 ? int64_t(t.rows) * wps * 8 : 0) + int64_t(t.rounds) * groups * 4;
+        if (best > 0.0 && cost >= best) continue;
+        if (!fit_lds(t, extra, 5, kGridElems<true>, 3, kGridElems<false>)) continue;
+        best = cost;
+        g = t;
+    }
+    return best > 0.0;
+}
+
+// Shape of a CSR grid: at least 64 rows per block
+bool shape_csr(grid_shape& g, int64_t n, int units)
+{
+    int64_t const most = std::min(units, kGridMaxBlocks);
+    int64_t rows = std::max<int64_t>(64, (n + most - 1) / most);
+    rows = (rows + 15) / 16 * 16;
+    if (rows > kGridThreads * kGridElems<false>) return false;
+    g.n = n;
+    g.rows = int32_t(rows);
+    g.blocks = int32_t((n + rows - 1) / rows);
+    return fit_lds(g, kCsrChunk * 8 + 4 * (rows + 1), 5, kGridElems<true>, 3, kGridElems<false>);
+}
+
+template <typename K>
+void allow_lds(K kernel, int64_t bytes)
+{
+    NEON_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       int(bytes)));
+}
+
+sym_matrix sym_of(linear_operator const& A)
+{
+    return sym_matrix{A.nodes,     A.slices,   A.sym_slots,
+                      A.sym_records, A.sym_sched, A.sym_rdiag,
+                      A.sym_eptr,  reinterpret_cast<const int4v*>(A.sym_ent),
+                      A.sym_rslice, A.sym_roff};
+}
+
+sell_matrix sell_of(linear_operator const& A)
+{
+    return sell_matrix{A.nodes, A.slices, A.sptr, A.snode, A.slane, A.scode, A.sexc, A.soff16, A.soff32};
+}
+} // namespace
+
+void krylov_engine::grid_begin()
+{
+    if (grid_units_) return;
+    NEON_CHECK_HIP(hipGetDevice(&grid_device_));
+    int units = 0;
+    NEON_CHECK_HIP(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, grid_device_));
+    grid_slots_.resize(2 * size_t(kGridMaxBlocks) * kGridSlotWords);
+    grid_clear();
+    grid_units_ = grid_device_ < unit_pool::kDevices ? units : 0;
+}
+
+void krylov_engine::grid_clear()
+{
+    fill_zero(s_, int64_t(grid_slots_.size()), reinterpret_cast<double*>(grid_slots_.data()));
+    fill_zero(s_, 2 * sizeof(krylov_state) / sizeof(double), reinterpret_cast<double*>(state_.data() + 2));
+    grid_epoch_ = 1;
+}
+
+// The link for one launch of at most `exchanges` exchanges
+grid_link krylov_engine::grid_next(uint32_t exchanges)
+{
+    if (grid_epoch_ > UINT32_MAX - exchanges - 1) grid_clear();
+    grid_link const l{grid_slots_.data(), state_.data() + 3, grid_patience, grid_epoch_};
+    grid_epoch_ += exchanges;
+    return l;
+}
+
+// Runs the launches of a resident grid: batch(true) starts the solve, batch(false) continues it
+// from the state in state_[2], whose copies the host reads one launch behind (launches past the
+// end return at once).  host_state_ holds the final state; false when the grid gave up (the
+// state and vectors are then worthless).
+template <typename Batch>
+bool krylov_engine::grid_run(Batch&& batch)
+{
+    auto step = [&](bool first, int slot) {
+        batch(first);
+        NEON_CHECK_HIP(hipGetLastError());
+        NEON_CHECK_HIP(hipMemcpyAsync(host_ring_ + 2 * slot, state_.data() + 2, 2 * sizeof(krylov_state),
+                                      hipMemcpyDeviceToHost, s_));
+        NEON_CHECK_HIP(hipEventRecord(ring_events_[slot], s_));
+    };
+    step(true, 0);
+    int wait = 0;
+    for (;; wait ^= 1)
+    {
+        step(false, wait ^ 1);
+        NEON_CHECK_HIP(hipEventSynchronize(ring_events_[wait]));
+        if (host_ring_[2 * wait].done || host_ring_[2 * wait + 1].done) break;
+    }
+    *host_state_ = host_ring_[2 * wait];
+    if (!host_ring_[2 * wait + 1].done && host_state_->done != KRYLOV_ABORTED) return true;
+    NEON_CHECK_HIP(hipStreamSynchronize(s_));
+    grid_clear();
+    return false;
+}
+
+bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion,
+                              double tol, int32_t max_it, const krylov_work* work, solve_result& out)
+{
+    if (prof && prof->enabled) return false; // per-launch timing needs the launches
+    grid_begin();
+    if (!grid_units_ || A.blocks_override > 0) return false;
+    grid_shape g;
+    bool ok = false;
+    if (A.node_block && A.sym)
+        ok = shape_sliced(g, A.n, A.sym_slots / 8, 1.0 + A.sym_mean, 1 + A.sym_entries, grid_units_);
+    else if (A.node_block && A.sell)
+        ok = shape_sliced(g, A.n, (A.slices + 7) / 8, A.sell_mean, A.sell_steps, grid_units_);
+    else if (!A.node_block)
+        ok = shape_csr(g, A.n, grid_units_);
+    if (!ok) return false;
+
+    int64_t const n = A.n;
+    int64_t const stride = (n + 31) / 32 * 32; // whole 128-byte lines
+    double *r = nullptr, *ring = nullptr;
+    int64_t buffers = 0;
+    if (work)
+    {
+        r = work->r;
+        ring = work->ring;
+        buffers = work->ring_size / stride;
+    }
+    else
+    {
+        grid_r_.reserve(stride);
+        buffers = std::clamp<int64_t>(kGridRing / stride, 8, 128);
+        grid_ring_.reserve(buffers * stride);
+        r = grid_r_.data();
+        ring = grid_ring_.data();
+    }
+    // small blocks: two exchanges and two ring buffers per iteration
+    bool const few = A.node_block ? g.wps > 1 && g.rounds == 1 : g.rows <= 256;
+    int const iters = int(std::min<int64_t>(few ? buffers / 2 : buffers, 64));
+    if (iters < 1) return false;
+    krylov_state* st = state_.data() + 2;
+    unit_hold const hold(grid_device_, g.blocks, grid_units_);
+    auto launch = [&](auto kernel, auto rows) {
+        allow_lds(kernel, g.lds);
+        return grid_run([&, kernel](bool first) {
+            kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, first ? b : nullptr, x, r, minv,
+                                                                  st, grid_next(uint32_t(3 * iters + 2)), iters,
+                                                                  criterion, tol, max_it);
+        });
+    };
+    auto with = [&](auto rows) {
+        if (few) return launch(cg_grid_small_kernel<decltype(rows)>, rows);
+        if (g.all) return launch(cg_grid_kernel<decltype(rows), true>, rows);
+        return launch(cg_grid_kernel<decltype(rows), false>, rows);
+    };
+    bool done = false;
+    if (A.sym)
+    {
+        using lay = grid_sym<double>;
+        lay const l{sym_of(A), A.s64};
+        int const items = (1 + A.sym_entries + g.wps - 1) / g.wps; // of a wavefront
+        if (few && g.wps == 8 && items <= 2)
+            done = launch(cg_grid_small_kernel<grid_kept<lay, 2, 8>>, grid_kept<lay, 2, 8>{{l}, {}});
+        else if (few && g.wps == 8 && items <= 4)
+            done = launch(cg_grid_small_kernel<grid_kept<lay, 4, 8>>, grid_kept<lay, 4, 8>{{l}, {}});
+        else if (few && g.wps == 4 && items <= 4)
+            done = launch(cg_grid_small_kernel<grid_kept<lay, 4, 4>>, grid_kept<lay, 4, 4>{{l}, {}});
+        else
+            done = with(grid_sliced<lay>{l});
+    }
+    else if (A.sell)
+    {
+        using lay = grid_sell<double>;
+        lay const l{sell_of(A), A.s64};
+        int const items = (A.sell_steps + g.wps - 1) / g.wps;
+        if (few && g.wps == 8 && items <= 4)
+            done = launch(cg_grid_small_kernel<grid_kept<lay, 4, 8>>, grid_kept<lay, 4, 8>{{l}, {}});
+        else if (few && g.wps == 4 && items <= 8)
+            done = launch(cg_grid_small_kernel<grid_kept<lay, 8, 4>>, grid_kept<lay, 8, 4>{{l}, {}});
+        else
+            done = with(grid_sliced<lay>{l});
+    }
+    else
+        done = with(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}});
+    if (!done) return false;
+    out = finish_solve(*host_state_, criterion);
+    out.spmv = out.iterations + (criterion == NEON_STOP_RELATIVE && host_state_->done == KRYLOV_CONVERGED ? 1 : 0);
+    return true;
+}
+} // namespace neon_amd

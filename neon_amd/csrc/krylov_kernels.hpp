@@ -10,60 +10,12 @@
 // with every scalar kept on the device (the CUDA code synchronises on each cuBLAS dot).
 #pragma once
 
-#include "common.hpp"
-#include "neon_hip.h"
+#include "spmv_layouts.hpp"
 
 #include <cfloat>
-#include <type_traits>
 
 namespace neon_amd
 {
-// Scalars of one Krylov iteration, ping-ponged between two device slots so that the
-// kernel that computes iteration k+1's scalars never overwrites what others still read.
-struct krylov_state
-{
-    double rz;        // r . z  (Eigen's absNew, CUDA's "residual")
-    double rr;        // r . r
-    double rhs2;      // b . b
-    double threshold; // Eigen: max(tol^2 ||b||^2, DBL_MIN)
-    double alpha, beta, omega, rho; // BiCGSTAB scalars (alpha reused by CG for reports)
-    double aux0, aux1;               // reliable-update bookkeeping (mixed precision)
-    int32_t it;   // iterations as the reference counts them
-    int32_t done; // 0 running, 1 converged, 2 iteration limit, 3 non-finite, 4 breakdown
-    int32_t restarts;
-    int32_t refine; // mixed precision: a reliable update is due this iteration
-};
-
-enum : int32_t
-{
-    KRYLOV_RUNNING = 0,
-    KRYLOV_CONVERGED = 1,
-    KRYLOV_LIMIT = 2,
-    KRYLOV_NONFINITE = 3,
-    KRYLOV_BREAKDOWN = 4,
-    KRYLOV_REFINE = 5, // mixed precision: a reliable update is due
-};
-
-// ----------------------------------------------------------------- SpMV layouts
-// Node-block CSR: the tangent of a 3-dof-per-node mesh keeps its values in ordinary
-// row-major CSR order (sorted columns), but every dof row of node n has the same column set
-// {3m+j : m in adj(n), j < 3}, so the kernels read one int32 block column per 9 values:
-//   row 3n+i, block s (node m = bcol[bptr[n]+s]), column 3m+j
-//   -> val[9 bptr[n] + i (3 deg n) + 3 s + j].
-struct nb_matrix
-{
-    int32_t nodes;
-    const int32_t* bptr;
-    const int32_t* bcol;
-};
-
-struct csr_matrix
-{
-    int32_t rows;
-    const int32_t* rp;
-    const int32_t* ci;
-};
-
 template <bool NT, typename T>
 __device__ inline T ld(const T* p)
 {
@@ -194,47 +146,6 @@ __global__ __launch_bounds__(kBlock) void spmv_nb_kernel(nb_matrix A, const VT* 
         if (threadIdx.x == 0) part[blockIdx.x] = dot;
     }
 }
-
-// Sliced node-block layout: a copy of the node-block values in which every wavefront load
-// reads one contiguous span.  Slice s holds the 64 consecutive nodes 64 s ... 64 s + 63 (lane l:
-// node snode[64 s + l]; an empty lane past the last node, snode -1 - m, gathers like node m and
-// holds zero values) and sptr[s+1] - sptr[s] steps, the largest block count among them; step kk
-// of a node is its kk-th block (ascending column node, as in bcol), and steps past a node's
-// block count hold zero values.  The 9 values of a step form one record of 9 x 64 values:
-// value t = 3 i + j of lane l sits at
-//   sval[576 (sptr[s] + kk) + sell_pos<VT>(t, l)]:
-// the first 8 in groups of W = 16 / sizeof(VT) per lane (one 16-byte load per lane and group;
-// group g spans 64 W values), the ninth after them (one value per lane).
-// A step's column offsets (column node - lane node): scode[step] < 0 encodes one offset shared
-// by the slice's lanes (shared_offset()) except at most two exception lanes, named by
-// slane[s] (8 bits each, 0xff for none), whose 16-bit offsets are in sexc[step]; scode[step]
-// >= 0 indexes 64 per-lane offsets at soff16 / soff32 [scode * 64 + lane].  A slice's steps
-// are all of one kind (the product tests the first code of each chunk of 64 steps).
-template <typename VT>
-__host__ __device__ constexpr int sell_pos(int t, int lane)
-{
-    constexpr int W = 16 / int(sizeof(VT));
-    return t < 8 ? (t / W) * 64 * W + lane * W + t % W : 512 + lane;
-}
-
-struct sell_matrix
-{
-    int32_t nodes;
-    int32_t slices;
-    const int32_t* sptr;   // [slices + 1] first step of each slice
-    const int32_t* snode;  // [slices * 64] node of each lane (-1 - m: empty lane gathering like node m)
-    const int32_t* slane;  // [slices] exception lanes of a slice's shared steps (8 bits each, 0xff: none)
-    const int32_t* scode;  // [steps] shared_code(offset) or the step's index into the per-lane offsets
-    const int32_t* sexc;   // [steps] 16-bit offsets of the exception lanes (shared steps)
-    const int16_t* soff16; // per-lane offsets when every one fits 16 bits (else null)
-    const int32_t* soff32; // per-lane offsets in 32 bits (used when soff16 is null)
-};
-constexpr int64_t kSharedBias = int64_t(1) << 30;
-__host__ __device__ inline int32_t shared_code(int64_t offset)
-{
-    return int32_t(int64_t(INT32_MIN) + kSharedBias + offset);
-}
-__host__ __device__ inline int64_t shared_offset(int32_t code) { return int64_t(code) - INT32_MIN - kSharedBias; }
 
 // y = A x on the sliced layout, one wavefront per slice, one node (three rows) per lane.  Each
 // lane accumulates its three row sums over its steps in order, so no cross-lane reduction is
@@ -479,42 +390,7 @@ __global__ __launch_bounds__(256) void sell_pack_lds_kernel(sell_matrix A, const
     }
 }
 
-// ------------------------------------------------ symmetric sliced layout
-// For a symmetric tangent the copy keeps the diagonal block and the upper blocks (column node -
-// row node = o > 0) only.  Slice s holds nodes 64 s .. 64 s + 63 (one per lane); its records of
-// 9 x 64 values (sell_pos layout) are the diagonal block (record rdiag[s]) and one record per
-// offset o in the slice's direct list (the upper offsets of its lanes' nodes): lane l's block
-// (i, i + o), zero where node i has no such neighbour.  The product adds, for every lane node i,
-// K(i, i + o) x(i + o) for the direct offsets and the transpose of K(i - o, i) x(i - o) for the
-// slice's lower offsets (those of its lanes' lower neighbours): that block is lane (i - o) % 64
-// of the record for o of slice (i - o) / 64, which is one of the two slices floor((64 s - o) /
-// 64) and the next one, whose record indices the entry carries.  Every off-diagonal value is
-// read twice, and the schedule makes the second read follow the first closely enough to be
-// served by the L2.  A slice's entries merge the two lists by offset, each {o, direct record or
-// -1, record in slice floor((64 s - o) / 64) or -1, record in the next slice or -1}, so that the
-// direct and the transposed read of one offset are issued together.
-// Schedule: wave slot q (workgroup q / 4, on XCD (q / 4) % 8) takes slice sched[q] (-1: none).
-// The host orders the slices in tiles (a band of the in-plane index, then plane by plane) and
-// gives each XCD one contiguous eighth of that order, so a slice's neighbours one plane down
-// were read on the same XCD a few workgroups earlier.
-constexpr int kMaxSymEntries = 40; // <= 64: a slice's entries fit one wavefront's lanes
-typedef int int4v __attribute__((ext_vector_type(4)));
-struct sym_matrix
-{
-    int32_t nodes;
-    int32_t slices;
-    int32_t slots;          // wave slots of the schedule (a multiple of 32)
-    int64_t records;        // records of the copy
-    const int32_t* sched;   // [slots] slice of each wave slot, -1 for none
-    const int32_t* rdiag;   // [slices] record of each slice's diagonal block
-    const int32_t* eptr;    // [slices + 1] entry range of each slice
-    const int4v* ent;       // entries, by slice and ascending offset
-    const int32_t* rslice;  // [records] slice of each record (packing)
-    const int32_t* roff;    // [records] offset of each record, 0 for the diagonal (packing)
-};
-
-// y = A x on the symmetric sliced layout (DOT, MODE, gate as in spmv_sell_kernel).  FP32
-// accumulation rotates over four accumulator sets as there; FP64 uses one.
+// y = A x on the symmetric sliced layout (DOT, MODE, gate as in spmv_sell_kernel).
 template <typename VT, typename XT, typename YT, typename AT, bool DOT, int MODE>
 __global__ __launch_bounds__(256) void spmv_sym_kernel(sym_matrix A, const VT* __restrict__ val,
                                                        const XT* __restrict__ x, YT* __restrict__ y,
@@ -525,27 +401,6 @@ __global__ __launch_bounds__(256) void spmv_sym_kernel(sym_matrix A, const VT* _
     int const lane = threadIdx.x & 63;
     int32_t const wave = __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x >> 6));
     int64_t const nodes = A.nodes;
-    constexpr int W = 16 / int(sizeof(VT));
-    typedef VT vec_t __attribute__((ext_vector_type(W)));
-    // the 9 values of lane l of the record at rec (NT: nontemporal, for a record read once)
-    auto load_rec = [&](const VT* rec, int l, VT(&v)[9], auto nt) {
-#pragma unroll
-        for (int g = 0; g < 8 / W; ++g)
-        {
-            const vec_t* src = reinterpret_cast<const vec_t*>(rec + g * 64 * W) + l;
-            vec_t q;
-            if constexpr (decltype(nt)::value)
-                q = __builtin_nontemporal_load(src);
-            else
-                q = *src;
-#pragma unroll
-            for (int j = 0; j < W; ++j) v[g * W + j] = q[j];
-        }
-        if constexpr (decltype(nt)::value)
-            v[8] = __builtin_nontemporal_load(rec + 512 + l);
-        else
-            v[8] = rec[512 + l];
-    };
     double dot = 0.0;
     for (int32_t q = int32_t(blockIdx.x) * 4 + wave; q < A.slots; q += int32_t(gridDim.x) * 4)
     {
@@ -553,9 +408,7 @@ __global__ __launch_bounds__(256) void spmv_sym_kernel(sym_matrix A, const VT* _
         if (s < 0) continue;
         int64_t const i = int64_t(s) * 64 + lane;
         bool const ok = i < nodes;
-        int64_t const ic = ok ? i : nodes - 1;
-        int64_t const row = 3 * ic;
-        int64_t const rdiag = A.rdiag[s];
+        int64_t const row = 3 * (ok ? i : nodes - 1);
         double br0 = 0.0, br1 = 0.0, br2 = 0.0;
         if constexpr (MODE == 1)
         {
@@ -564,96 +417,8 @@ __global__ __launch_bounds__(256) void spmv_sym_kernel(sym_matrix A, const VT* _
             br2 = bvec[row + 2];
         }
         XT const xo0 = x[row], xo1 = x[row + 1], xo2 = x[row + 2];
-        AT a0 = AT(0), a1 = AT(0), a2 = AT(0), b0 = AT(0), b1 = AT(0), b2 = AT(0);
-        AT c0 = AT(0), c1 = AT(0), c2 = AT(0), d0 = AT(0), d1 = AT(0), d2 = AT(0);
-        // one block's product (transposed: K^T x) into the next accumulator set
-        auto accumulate = [&](VT const(&v)[9], XT x0_, XT x1_, XT x2_, bool tr) {
-            AT const x0 = AT(x0_), x1 = AT(x1_), x2 = AT(x2_);
-            AT n0, n1, n2;
-            if (tr)
-            {
-                n0 = a0 + (AT(v[0]) * x0 + AT(v[3]) * x1 + AT(v[6]) * x2);
-                n1 = a1 + (AT(v[1]) * x0 + AT(v[4]) * x1 + AT(v[7]) * x2);
-                n2 = a2 + (AT(v[2]) * x0 + AT(v[5]) * x1 + AT(v[8]) * x2);
-            }
-            else
-            {
-                n0 = a0 + (AT(v[0]) * x0 + AT(v[1]) * x1 + AT(v[2]) * x2);
-                n1 = a1 + (AT(v[3]) * x0 + AT(v[4]) * x1 + AT(v[5]) * x2);
-                n2 = a2 + (AT(v[6]) * x0 + AT(v[7]) * x1 + AT(v[8]) * x2);
-            }
-            if constexpr (sizeof(AT) == 4)
-            {
-                a0 = b0, a1 = b1, a2 = b2;
-                b0 = c0, b1 = c1, b2 = c2;
-                c0 = d0, c1 = d1, c2 = d2;
-                d0 = n0, d1 = n1, d2 = n2;
-            }
-            else
-            {
-                a0 = n0, a1 = n1, a2 = n2;
-            }
-        };
-        {
-            VT v[9];
-            load_rec(val + rdiag * 576, lane, v, std::true_type{});
-            accumulate(v, xo0, xo1, xo2, false);
-        }
-        // one entry's operands: the stored block K(i, i + o) and x(i + o) (zero where the slice
-        // has no direct record for o), and the transpose of K(i - o, i) and x(i - o) (x counts
-        // as zero where node i - o does not exist or holds no block for o: its values are then
-        // read from the slice's own diagonal record, in bounds)
-        int32_t const e0 = A.eptr[s], ne = A.eptr[s + 1] - e0;
-        // the slice's entries (at most kMaxSymEntries <= 64), lane k holding entry k: one
-        // coalesced load, then each entry read from its lane (no scalar-load wait in the loop)
-        int4v const mine = lane < ne ? A.ent[e0 + lane] : int4v{0, 0, -1, -1};
-        struct pair_t
-        {
-            VT v[9], w[9];
-            XT x0, x1, x2, z0, z1, z2;
-            bool dv, jv;
-        };
-        auto fetch = [&](int32_t m) {
-            pair_t o;
-            int4v const e{__builtin_amdgcn_readlane(mine.x, m), __builtin_amdgcn_readlane(mine.y, m),
-                          __builtin_amdgcn_readlane(mine.z, m), __builtin_amdgcn_readlane(mine.w, m)};
-            int64_t const off = e.x;
-            int64_t const rd = e.y;
-            o.dv = rd >= 0;
-            int64_t const mi = i + off < nodes ? i + off : nodes - 1;
-            load_rec(val + (o.dv ? rd : rdiag) * 576, lane, o.v, std::false_type{});
-            o.x0 = x[3 * mi], o.x1 = x[3 * mi + 1], o.x2 = x[3 * mi + 2];
-            int64_t const j0 = i - off;
-            int64_t const sa = (int64_t(s) * 64 - off) >> 6; // floor division by 64
-            int64_t const rt = (j0 >> 6) == sa ? int64_t(e.z) : int64_t(e.w);
-            o.jv = j0 >= 0 && j0 < nodes && rt >= 0;
-            int64_t const j = o.jv ? j0 : ic;
-            load_rec(val + (o.jv ? rt : rdiag) * 576, o.jv ? int(j & 63) : lane, o.w, std::false_type{});
-            o.z0 = x[3 * j], o.z1 = x[3 * j + 1], o.z2 = x[3 * j + 2];
-            return o;
-        };
-        auto accumulate_pair = [&](pair_t const& o) {
-            accumulate(o.v, o.dv ? o.x0 : XT(0), o.dv ? o.x1 : XT(0), o.dv ? o.x2 : XT(0), false);
-            accumulate(o.w, o.jv ? o.z0 : XT(0), o.jv ? o.z1 : XT(0), o.jv ? o.z2 : XT(0), true);
-        };
-        // software-pipelined over two register sets: entry m + 1's loads are issued before
-        // entry m is accumulated (3 % faster at 128^3 in both precisions than a plain loop)
-        int32_t m = 0;
-        if (ne >= 2)
-        {
-            pair_t sa_ = fetch(0);
-            for (; m + 2 < ne; m += 2)
-            {
-                pair_t const sb = fetch(m + 1);
-                accumulate_pair(sa_);
-                sa_ = fetch(m + 2);
-                accumulate_pair(sb);
-            }
-            accumulate_pair(sa_);
-            m += 1;
-        }
-        for (; m < ne; ++m) accumulate_pair(fetch(m));
-        AT const r0 = (a0 + b0) + (c0 + d0), r1 = (a1 + b1) + (c1 + d1), r2 = (a2 + b2) + (c2 + d2);
+        AT r0, r1, r2;
+        sym_slice_rows<1, VT, XT, AT>(A, val, x, sym_load_head(A, s, lane), lane, 0, false, xo0, xo1, xo2, r0, r1, r2);
         YT const y0 = MODE == 1 ? YT(br0 - double(r0)) : YT(r0);
         YT const y1 = MODE == 1 ? YT(br1 - double(r1)) : YT(r1);
         YT const y2 = MODE == 1 ? YT(br2 - double(r2)) : YT(r2);
@@ -847,26 +612,7 @@ __global__ __launch_bounds__(kBlock) void cg_init_state_kernel(const double* __r
 {
     double const rr = reduce_partials<kBlock>(part_rr, npart);
     double const rz = reduce_partials<kBlock>(part_rz, npart);
-    if (threadIdx.x != 0) return;
-    krylov_state s{};
-    s.rz = rz;
-    s.rr = rr;
-    s.rhs2 = rr;
-    s.it = 0;
-    s.done = KRYLOV_RUNNING;
-    if (criterion == NEON_STOP_RELATIVE)
-    {
-        s.threshold = fmax(tol * tol * rr, DBL_MIN);
-        if (rr == 0.0 || rr < s.threshold) s.done = KRYLOV_CONVERGED;
-    }
-    else
-    {
-        s.threshold = 0.0;
-        if (!(sqrt(rz) > tol)) s.done = KRYLOV_CONVERGED;
-    }
-    if (s.done == KRYLOV_RUNNING && max_it <= 0) s.done = KRYLOV_LIMIT;
-    if (!isfinite(rr) || !isfinite(rz)) s.done = KRYLOV_NONFINITE;
-    *st = s;
+    if (threadIdx.x == 0) *st = cg_first_state(rr, rz, criterion, tol, max_it);
 }
 
 // x += alpha p, r -= alpha Ap with alpha = rz / (p.Ap); partials of r.r and r.z
@@ -984,28 +730,8 @@ __global__ __launch_bounds__(kBlock) void cg_update_p_kernel(int64_t n, double* 
     double const alpha = s.rz / partials_total<kBlock>(part_pAp, -1);
     double const rr = partials_total<kBlock>(part_rr, npart);
     double const rz = partials_total<kBlock>(part_rz, npart);
-    int32_t it_new;
-    int32_t done = KRYLOV_RUNNING;
-    if (criterion == NEON_STOP_RELATIVE)
-    {
-        bool const conv = rr < s.threshold; // Eigen breaks before counting the iteration
-        it_new = conv ? s.it : s.it + 1;
-        if (conv)
-            done = KRYLOV_CONVERGED;
-        else if (it_new >= max_it)
-            done = KRYLOV_LIMIT;
-    }
-    else
-    {
-        it_new = s.it + 1; // the CUDA loop counts at the top
-        if (it_new >= max_it)
-            done = KRYLOV_LIMIT;
-        else if (!(sqrt(rz) > tol))
-            done = KRYLOV_CONVERGED;
-    }
-    if (!isfinite(rr) || !isfinite(rz)) done = KRYLOV_NONFINITE;
-    double const beta = rz / s.rz;
-    bool const more = done == KRYLOV_RUNNING;
+    double const beta = cg_decide(s, rr, rz, criterion, tol, max_it);
+    bool const more = s.done == KRYLOV_RUNNING;
     int64_t beg, end;
     xcd_chunk_aligned<2>(n, beg, end);
     int64_t const full = beg + (end - beg) / 2 * 2;
@@ -1027,17 +753,8 @@ __global__ __launch_bounds__(kBlock) void cg_update_p_kernel(int64_t n, double* 
         x[i] = x[i] + alpha * pi;
         if (more) p[i] = minv[i] * r[i] + beta * pi;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        s.rr = rr;
-        s.rz = rz;
-        s.beta = beta;
-        s.it = it_new;
-        s.done = done;
-        *st_next = s;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *st_next = s;
 }
-
 
 // ------------------------------------------------------------- BiCGSTAB (FP64)
 // Device-resident right-preconditioned BiCGSTAB: every scalar stays in one krylov_state, which

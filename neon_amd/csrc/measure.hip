@@ -266,4 +266,16 @@ int neon_stream_probe(neon_context* ctx, int64_t bytes, int32_t reps, double* re
     });
 }
 
+// How long the workgroups of a solver's resident grid wait for each other before the solve falls
+// back to launches (ticks of 10 ns; 0: a wait that has to wait at all gives up).  Not a probe and not
+// in the header: the fallback's test sets it.
+int neon_test_grid_patience(neon_context* ctx, int64_t ticks)
+{
+    return measured(ctx, [&] {
+        if (ticks < 0) throw status_error(NEON_BAD_ARGUMENT, "negative patience");
+        ctx->engine->grid_patience = uint64_t(ticks);
+        return NEON_OK;
+    });
+}
+
 } // extern "C"

@@ -1,0 +1,208 @@
+"""The Krylov loops inside one resident grid (neon_amd/csrc/grid_kernels.hpp) at the sizes where
+their layouts can go wrong, against the launch-per-phase loops (which a solve takes while kernel
+timing is on) and the true residual of the downloaded or host matrix.
+
+Tolerances: both loops stop on a recurrence residual of 1e-10 |b|; the true residual differs from
+it by the rounding of the recurrence, some eps |A| |x| per iteration, below 1e-11 |b| on these
+systems (condition below 1e5), so it is held to 1.1e-10 |b|.  The iteration counts differ only where
+the last residual lands within rounding of the tolerance: 2 or 2 %, as for the oracle's counts."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import neon_amd
+from neon_amd import _capi, problems
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(ctx, solve):
+    """solve() on the resident grid and by launches."""
+    grid = solve()
+    ctx.profile(True)
+    try:
+        launches = solve()
+    finally:
+        ctx.profile(False)
+    return grid, launches
+
+
+def _check(A, b, grid, launches):
+    for x, its, _ in (grid, launches):
+        res = np.linalg.norm(b - A @ x) / np.linalg.norm(b)
+        assert res <= 1.1e-10, res
+    assert abs(grid[1] - launches[1]) <= max(2, 0.02 * launches[1]), (grid[1], launches[1])
+
+
+# One to three slices; the last with one node; eight wavefronts per slice with two and four items
+# each; four per slice; several rounds; one wavefront per slice; two rounds of it; and the rows too
+# many for every vector to stay in LDS.  The plates' slices have up to 31 entries, the generated
+# numbering none of the common offsets (the full copy).
+MESHES = [((1, 1, 1), "grid", 0.0), ((3, 3, 3), "grid", 0.0), ((4, 4, 4), "grid", 0.0), ((12, 4, 4), "grid", 0.0),
+          ((20, 21, 19), "grid", 0.0), ((29, 31, 30), "grid", 0.0), ((35, 33, 34), "grid", 0.0),
+          ((43, 40, 41), "grid", 0.0), ((52, 50, 51), "grid", 0.0), ((66, 65, 64), "grid", 0.0),
+          ((24, 12, 6), "grid", 1.5), ((64, 32, 20), "grid", 4.0),
+          ((5, 4, 6), "shuffled", 0.0), ((23, 22, 24), "shuffled", 0.0), ((31, 30, 33), "boundary", 0.0),
+          ((45, 44, 46), "boundary", 0.0)]
+
+
+def _mesh(ctx, dims, numbering, hole):
+    if hole:
+        p = problems.notched_plate_j2(*dims, hole_cells=hole)
+        model = neon_amd.MODEL_LINEAR_ELASTIC
+    else:
+        p = problems.block_rollers(max(dims), dims=dims)
+        model = p.model
+    X, conn, ijk, fixed = p.X, p.conn, p.ijk, p.fixed_dofs()
+    if numbering != "grid":
+        if numbering == "shuffled":
+            order = np.random.default_rng(3).permutation(len(X))
+        else:
+            faces = np.sum((ijk == 0) | (ijk == np.array(dims)), axis=1)
+            order = np.argsort(-faces, kind="stable")
+        new = np.empty(len(order), np.int32)
+        new[order] = np.arange(len(order), dtype=np.int32)
+        X, conn = X[order], new[conn]
+        fixed = np.sort(3 * new[fixed // 3] + fixed % 3).astype(np.int32)
+    mg = neon_amd.DeviceMesh(X, conn, p.params, model=model, context=ctx)
+    mg.update_internal_variables()
+    mg.assemble()
+    b = np.random.default_rng(11).standard_normal(mg.n_dofs)
+    mg.enforce_dirichlet(fixed, b)
+    return mg, b
+
+
+def _matrix(mg):
+    rp, ci = mg.pattern()
+    val, _ = mg.download(internal_force=False)
+    return sp.csr_matrix((val, ci, rp))
+
+
+@pytest.mark.parametrize("dims,numbering,hole", MESHES)
+def test_cg_on_the_mesh_tangent(ctx, dims, numbering, hole):
+    print(dims, numbering, hole, flush=True)
+    mg, b = _mesh(ctx, dims, numbering, hole)
+    grid, launches = _both(ctx, lambda: mg.solve(b, tol=1e-10))
+    _check(_matrix(mg), b, grid, launches)
+
+
+def test_cg_with_32bit_offsets(ctx):
+    mg, b = _mesh(ctx, (12, 11, 13), "shuffled", 0.0)
+    mg.spmv_config(flags=neon_amd.SPMV_SLICED | neon_amd.SPMV_INDEX32)
+    grid, launches = _both(ctx, lambda: mg.solve(b, tol=1e-10))
+    _check(_matrix(mg), b, grid, launches)
+
+
+def _spd(n, per_row, seed, long_rows=0):
+    """A diagonally dominant symmetric matrix of n rows with about per_row entries each, every
+    seventh row its diagonal alone, and long_rows rows that couple to every row."""
+    rng = np.random.default_rng(seed)
+    m = n * per_row // 2
+    i, j = rng.integers(0, n, m), rng.integers(0, n, m)
+    keep = (i % 7 != 0) & (j % 7 != 0) & (i != j)
+    i, j = i[keep], j[keep]
+    for r in range(long_rows):
+        i = np.concatenate([i, np.full(n - 1, n // 2 + r)])
+        j = np.concatenate([j, np.delete(np.arange(n), n // 2 + r)])
+    S = sp.coo_matrix((rng.uniform(-1, 1, len(i)), (i, j)), shape=(n, n)).tocsr()
+    S = S + S.T
+    S = (S + sp.diags(np.abs(S).sum(axis=1).A1 * 1.05 + 1.0)).tocsr()
+    S.sort_indices()
+    return S, rng.standard_normal(n)
+
+
+# one row; a block's 64 rows and one more; chunks of 4,096 entries with rows across their ends;
+# rows longer than a chunk; many blocks, all vectors in LDS and not
+CSR = [(1, 1, 0), (15, 3, 0), (64, 5, 0), (65, 5, 0), (1000, 90, 0), (6000, 12, 2), (16384, 6, 0), (70001, 30, 0),
+       (300007, 8, 0), (1200000, 4, 0)]
+
+
+def _solve_csr(ctx, cls, A, b, tol=1e-10, criterion=neon_amd.STOP_RELATIVE):
+    s = cls(tol, 4000, criterion=criterion, context=ctx)
+    x = np.zeros(len(b))
+    s.solve(A, x, b)
+    return x, s.iterations, s.error
+
+
+@pytest.mark.parametrize("n,per_row,long_rows", CSR)
+def test_cg_on_host_csr(ctx, n, per_row, long_rows):
+    print(n, per_row, long_rows, flush=True)
+    A, b = _spd(n, per_row, n, long_rows)
+    grid, launches = _both(ctx, lambda: _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b))
+    _check(A, b, grid, launches)
+
+
+@pytest.mark.parametrize("criterion", [neon_amd.STOP_RELATIVE, neon_amd.STOP_ABSOLUTE_PRECONDITIONED])
+def test_cg_ends(ctx, criterion):
+    """A zero right-hand side, the iteration limit inside and at the end of a launch, and values
+    that are not finite end as they do by launches."""
+    mg, b = _mesh(ctx, (12, 4, 4), "grid", 0.0)
+    solve = dict(criterion=criterion, tol=1e-30)
+    x, its, err = mg.solve(np.zeros_like(b), **solve)
+    assert its == 0 and err == 0.0 and not x.any()
+    A = _matrix(mg)
+    for limit in (1, 63, 64, 65):
+        outcomes = []
+        for timed in (False, True):
+            s = neon_amd.conjugate_gradient_hip(1e-30, limit, criterion=criterion, context=ctx)
+            x = np.zeros_like(b)
+            ctx.profile(timed)
+            try:
+                with pytest.raises(neon_amd.computational_error) as e:
+                    s.solve(A, x, b)
+            finally:
+                ctx.profile(False)
+            outcomes.append((e.value.code, s.iterations))
+        assert outcomes == [(_capi.NEON_NONCONVERGED, limit)] * 2
+    b[17] = np.inf
+    with pytest.raises(neon_amd.computational_error) as e:
+        mg.solve(b, **solve)
+    assert e.value.code == _capi.NEON_NAN_OR_INF
+
+
+def test_a_grid_that_gives_up_is_solved_by_launches(ctx):
+    """With no patience the first wait of a workgroup for another ends the grid; the solve then
+    takes the launch-per-phase loop, and the next one with patience the grid again."""
+    fn = _capi.measure_lib().neon_test_grid_patience
+    fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.c_int64]
+    A, b = _spd(40000, 20, 8)
+
+    def solve():
+        return _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b)
+
+    grid, launches = _both(ctx, solve)
+    ctx.check(fn(ctx.handle, 0))
+    try:
+        impatient = solve()
+    finally:
+        ctx.check(fn(ctx.handle, 10 ** 8))
+    assert np.array_equal(impatient[0], launches[0]) and impatient[1] == launches[1]
+    again = solve()
+    assert np.array_equal(again[0], grid[0]) and again[1] == grid[1]
+
+
+def test_two_contexts_share_the_gpu():
+    """Solves on two contexts from two threads at once: the grids take turns for the compute units."""
+    import threading
+
+    results = {}
+
+    def work(k):
+        c = neon_amd.Context(0)
+        try:
+            A, b = _spd(200000, 20, 30 + k)
+            results[k] = [_solve_csr(c, neon_amd.conjugate_gradient_hip, A, b)[0] for _ in range(3)]
+            results[k].append(np.linalg.norm(b - A @ results[k][0]) / np.linalg.norm(b))
+        finally:
+            c.close()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(2):
+        assert results[k][3] <= 1.1e-10
+        assert np.array_equal(results[k][0], results[k][1]) and np.array_equal(results[k][0], results[k][2])
