@@ -82,7 +82,7 @@ void launch_spmv(const linear_operator& A, hipStream_t s, const VT* val, const V
                            A.sym_records, A.sym_sched, A.sym_rdiag,
                            A.sym_eptr,  reinterpret_cast<const int4v*>(A.sym_ent),
                            A.sym_rslice, A.sym_roff};
-        spmv_sym_kernel<VT, XT, YT, AT, DOT, MODE><<<blocks, 256, 0, s>>>(m, sval, x, y, b, part, st, gate);
+        spmv_sym_kernel<VT, XT, YT, AT, DOT, MODE><<<blocks, 256, 0, s>>>(m, sval, x, y, b, part, st, gate, A.back);
         NEON_CHECK_HIP(hipGetLastError());
         return;
     }
@@ -91,7 +91,7 @@ void launch_spmv(const linear_operator& A, hipStream_t s, const VT* val, const V
         if (!sval) throw status_error(NEON_BAD_ARGUMENT, "sliced operator without sliced values");
         sell_matrix m{A.nodes, A.slices, A.sptr, A.snode, A.slane, A.scode, A.sexc, A.soff16, A.soff32};
 #define NEON_SELL(I16, NT) \
-    spmv_sell_kernel<I16, NT, VT, XT, YT, AT, DOT, MODE><<<blocks, 256, 0, s>>>(m, sval, x, y, b, part, st, gate)
+    spmv_sell_kernel<I16, NT, VT, XT, YT, AT, DOT, MODE><<<blocks, 256, 0, s>>>(m, sval, x, y, b, part, st, gate, A.back)
         if (A.nb_nt)
         {
             if (A.soff16)
@@ -373,13 +373,15 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
     NEON_CHECK_HIP(hipGetLastError());
 
     int64_t launched = 0;
+    linear_operator Ak = A; // its products alternate in order
     run_batches(st, launched, [&] {
         for (int k = 0; k < poll_every; ++k, ++launched)
         {
             krylov_state* cur = st + (launched & 1);
             krylov_state* nxt = st + ((launched + 1) & 1);
             int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP64) : -1;
-            A.apply64(s_, p, Ap, part_pAp, cur);
+            Ak.back = int(launched & 1);
+            Ak.apply64(s_, p, Ap, part_pAp, cur);
             if (prof) prof->end(s_, tok);
             totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
             cg_update_xr_kernel<<<nb, kBlock, 0, s_>>>(n, r, Ap, minv, part_pAp, -1, cur, part_rr, part_rz);
@@ -598,7 +600,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     // arithmetic; x64 stays unscaled (the folds scale the steps back) and the FP64 residuals
     // r = b - K x64 use A, the unscaled FP32 values, so convergence is judged on K as without it
     bool const scaled = minv64_scaled != nullptr;
-    linear_operator const& Arec = scaled ? *scaled_op : A;
+    linear_operator Ak = scaled ? *scaled_op : A; // its products alternate in order
     if (scaled)
         mixed_init_scaled_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv64_scaled, part_rr, part_rz);
     else
@@ -616,7 +618,8 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
             krylov_state* cur = st + (launched & 1);
             krylov_state* nxt = st + ((launched + 1) & 1);
             int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP32) : -1;
-            Arec.apply32(s_, p32, Ap32, part_pAp, cur);
+            Ak.back = int(launched & 1);
+            Ak.apply32(s_, p32, Ap32, part_pAp, cur);
             if (prof) prof->end(s_, tok);
             totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
             // the reliable-update / true-residual convergence test runs every refine_every

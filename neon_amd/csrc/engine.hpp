@@ -118,6 +118,8 @@ struct linear_operator
     int nb_lanes = 32;
     bool nb_nt = false;
     int blocks_override = 0;
+    // the sliced layouts' slices in the opposite order (spmv_sell_kernel)
+    int back = 0;
     // values
     const double* v64 = nullptr;
     const float* v32 = nullptr;
