@@ -283,9 +283,11 @@ int neon_krylov_solve_csr_noalloc(neon_context* ctx, int solver, int criterion, 
         for (int k = 0; k < 8; ++k) *slots[k] = vec + (k + 1) * kNoAllocRows;
         // BiCGSTAB's eighth vector: CG's Ap slot is free there
         w.s_hat = w.Ap;
-        // the resident grid's CG: all behind r
+        // the resident grids' rings: all behind r for CG, the last three vectors for BiCGSTAB
         w.ring = vec + 2 * kNoAllocRows;
         w.ring_size = 7 * kNoAllocRows;
+        w.bicg_ring = vec + 6 * kNoAllocRows;
+        w.bicg_ring_size = 3 * kNoAllocRows;
         ctx->engine->jacobi64(A, minv, criterion == NEON_STOP_RELATIVE ? 1 : 0);
         solve_result const r =
             solver == NEON_SOLVER_CG

@@ -398,6 +398,31 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
     return res;
 }
 
+solve_result finish_bicg(const krylov_state& f, int criterion)
+{
+    solve_result res;
+    res.iterations = f.it;
+    res.spmv = 2ll * f.it + f.restarts;
+    if (criterion == NEON_STOP_ABSOLUTE_PRECONDITIONED)
+    {
+        res.error = std::sqrt(f.rz);
+        switch (f.done)
+        {
+        case KRYLOV_CONVERGED: res.status = NEON_OK; break;
+        case KRYLOV_BREAKDOWN: res.status = NEON_BREAKDOWN; break;
+        case KRYLOV_NONFINITE: res.status = NEON_NAN_OR_INF; break;
+        default: res.status = NEON_NONCONVERGED; break;
+        }
+    }
+    else
+    {
+        res.error = f.rhs2 > 0.0 ? std::sqrt(f.rr / f.rhs2) : 0.0;
+        res.status = f.done == KRYLOV_NONFINITE ? NEON_NAN_OR_INF
+                                                : (f.done == KRYLOV_LIMIT ? NEON_NONCONVERGED : NEON_OK);
+    }
+    return res;
+}
+
 // Jacobi-BiCGSTAB in FP64 (the unsymmetric selection) with every scalar on the device and the
 // host polling the state like the CG loop (bicg_* kernels).  criterion
 // NEON_STOP_ABSOLUTE_PRECONDITIONED follows biconjugate_gradient_stabilised_cuda::solve
@@ -406,6 +431,8 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
 solve_result krylov_engine::bicgstab64(const linear_operator& A, const double* b, double* x, const double* minv,
                                        int criterion, double tol, int32_t max_it, const krylov_work* work)
 {
+    solve_result res;
+    if (bicgstab64_grid(A, b, x, minv, criterion, tol, max_it, work, res)) return res;
     int64_t const n = A.n;
     if (!work)
     {
@@ -442,33 +469,10 @@ solve_result krylov_engine::bicgstab64(const linear_operator& A, const double* b
     NEON_CHECK_HIP(hipMemsetAsync(v, 0, bytes, s_));
     NEON_CHECK_HIP(hipMemsetAsync(p, 0, bytes, s_));
     double const bb = dot(n, b, b);
-    krylov_state s0{};
-    s0.rz = bb; // r0 . r = b . b
-    s0.rr = bb;
-    s0.rhs2 = bb;
-    s0.aux0 = 1.0; // Eigen's rho_old, alpha, omega start at 1
-    s0.alpha = 1.0;
-    s0.omega = 1.0;
-    s0.aux1 = bb; // Eigen's |r0|^2
-    if (cuda_rule)
-    {
-        s0.aux0 = 0.0;
-        s0.alpha = s0.omega = 0.0;
-        if (!(std::sqrt(bb) > tol)) s0.done = KRYLOV_CONVERGED;
-        else if (max_it <= 0) s0.done = KRYLOV_LIMIT;
-    }
-    else
-    {
-        s0.threshold = tol * tol * bb;
-        if (bb == 0.0 || !(bb > s0.threshold)) s0.done = KRYLOV_CONVERGED;
-        else if (max_it <= 0) s0.done = KRYLOV_LIMIT;
-    }
-    if (!std::isfinite(bb)) s0.done = KRYLOV_NONFINITE;
-    *host_state_ = s0;
+    *host_state_ = bicg_first_state(bb, cuda_rule ? 1 : 0, tol, max_it);
     NEON_CHECK_HIP(hipMemcpyAsync(st, host_state_, sizeof(krylov_state), hipMemcpyHostToDevice, s_));
     // the state is a single slot (decision kernels write it between the grid kernels that read
     // it), so run_batches reads st[launched & 1] = st[0] with launched kept even
-    solve_result res;
     int64_t launched = 0;
     run_batches(st, launched, [&] {
         for (int k = 0; k < poll_every; ++k)
@@ -495,27 +499,8 @@ solve_result krylov_engine::bicgstab64(const linear_operator& A, const double* b
                                                      tol, max_it);
         }
     });
-    krylov_state const& f = *host_state_;
-    res.iterations = f.it;
-    res.spmv = 2ll * f.it + f.restarts;
-    if (prof) prof->collect(f.it);
-    if (cuda_rule)
-    {
-        res.error = std::sqrt(f.rz);
-        switch (f.done)
-        {
-        case KRYLOV_CONVERGED: res.status = NEON_OK; break;
-        case KRYLOV_BREAKDOWN: res.status = NEON_BREAKDOWN; break;
-        case KRYLOV_NONFINITE: res.status = NEON_NAN_OR_INF; break;
-        default: res.status = NEON_NONCONVERGED; break;
-        }
-    }
-    else
-    {
-        res.error = f.rhs2 > 0.0 ? std::sqrt(f.rr / f.rhs2) : 0.0;
-        res.status = f.done == KRYLOV_NONFINITE ? NEON_NAN_OR_INF
-                                                : (f.done == KRYLOV_LIMIT ? NEON_NONCONVERGED : NEON_OK);
-    }
+    res = finish_bicg(*host_state_, criterion);
+    if (prof) prof->collect(res.iterations);
     return res;
 }
 

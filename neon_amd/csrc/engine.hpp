@@ -169,9 +169,9 @@ struct krylov_work
 {
     double *r = nullptr, *p = nullptr, *Ap = nullptr;
     double *r0 = nullptr, *v = nullptr, *s = nullptr, *t = nullptr, *p_hat = nullptr, *s_hat = nullptr;
-    // the resident-grid loops' vectors instead: ring_size doubles, none of the above but r among them
-    double* ring = nullptr;
-    int64_t ring_size = 0;
+    // the resident-grid loops' rings: CG's beside r, BiCGSTAB's beside r, p, r0 and v (doubles)
+    double *ring = nullptr, *bicg_ring = nullptr;
+    int64_t ring_size = 0, bicg_ring_size = 0;
 };
 
 struct grid_link; // grid_kernels.hpp
@@ -179,6 +179,7 @@ struct grid_link; // grid_kernels.hpp
 // least 8 iterations' worth)
 constexpr int64_t kGridRing = int64_t(1) << 23;
 solve_result finish_solve(const krylov_state& s, int criterion);
+solve_result finish_bicg(const krylov_state& s, int criterion);
 
 class krylov_engine
 {
@@ -251,6 +252,8 @@ private:
     // gave up; the launch-per-phase loop then solves
     bool cg64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion, double tol,
                    int32_t max_it, const krylov_work* work, solve_result& out);
+    bool bicgstab64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion,
+                         double tol, int32_t max_it, const krylov_work* work, solve_result& out);
     void grid_begin();
     void grid_clear();
     grid_link grid_next(uint32_t exchanges);
@@ -259,7 +262,7 @@ private:
     int grid_device_ = 0, grid_units_ = 0;
     uint32_t grid_epoch_ = 1;
     device_array<uint64_t> grid_slots_;
-    device_array<double> grid_ring_, grid_r_;
+    device_array<double> grid_ring_, grid_r_, grid_bicg_;
     double* host_scalar_ = nullptr;
     device_array<double> scalar_;
     int64_t n_ = 0, n_mixed_ = 0;

@@ -1019,4 +1019,189 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_small_kernel(ROWS rows, 
         *st = s;
     }
 }
+
+// ------------------------------------------------------------------ BiCGSTAB
+// Up to `iters` iterations of bicgstab64's Jacobi-BiCGSTAB with both stopping rules (the recurrence
+// and scalars of the bicg_* kernels, the dot products summed in another fixed order): five
+// exchanges per iteration (one carries only p_hat) in place of nine to thirteen launches.
+// first: the launch starts the solve (x = 0, r = r0 = b, p = v = 0), else it continues the one in
+// *st.  Ring buffers 3 k, 3 k + 1 and 3 k + 2 take p_hat, s_hat and, at a restart of the Eigen rule,
+// x of the launch's iteration k.  All vectors are in LDS; x, r, r0, p and v leave through global
+// memory.
+constexpr int kGridBicgVectors = 8;
+template <typename ROWS>
+__global__ __launch_bounds__(kGridThreads) void bicg_grid_kernel(ROWS rows, grid_shape g, double* ring, int64_t stride,
+                                                                 const double* __restrict__ b, double* __restrict__ x,
+                                                                 double* __restrict__ r, double* __restrict__ r0,
+                                                                 double* __restrict__ p, double* __restrict__ v,
+                                                                 const double* __restrict__ minv, krylov_state* st,
+                                                                 grid_link link, int first, int iters, int cuda_rule,
+                                                                 double tol, int max_it)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ double own[2][2][kGridWaves], all[2][2][kGridWaves];
+    __shared__ int bad;
+    int const tid = threadIdx.x;
+    krylov_state s{};
+    if (!first)
+    {
+        s = *st;
+        if (s.done) return;
+    }
+    if (tid == 0) bad = __hip_atomic_load(&link.mark->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    double* const l_y = reinterpret_cast<double*>(smem); // a product's rows
+    double* const l_r = l_y + g.rows;                    // r, and s between the two products
+    double* const l_r0 = l_r + g.rows;
+    double* const l_p = l_r0 + g.rows;
+    double* const l_v = l_p + g.rows;
+    double* const l_x = l_v + g.rows;
+    double* const l_m = l_x + g.rows;
+    double* const l_b = l_m + g.rows;
+    double* const part = l_b + g.rows;
+    int32_t* const first_row =
+        reinterpret_cast<int32_t*>(part + (!ROWS::kSliced ? kCsrChunk : g.wps > 1 ? g.rows * g.wps : 0));
+    rows.begin(g, first_row);
+    __syncthreads();
+    grid_exchange ex{link, g.blocks, own, all, &bad};
+    if (bad)
+    {
+        if (blockIdx.x == 0 && tid == 0) st->done = KRYLOV_ABORTED;
+        return;
+    }
+    rows.hold(g, first_row);
+    // f(local row, row) over the thread's rows
+    auto each = [&](auto f) {
+        for (int lr = tid; lr < g.rows; lr += kGridThreads)
+        {
+            int64_t const i = rows.row(g, first_row, lr);
+            if (i >= 0) f(lr, i);
+        }
+    };
+    double d[2] = {0.0, 0.0};
+    each([&](int lr, int64_t i) {
+        double const bi = b[i];
+        l_b[lr] = bi;
+        l_m[lr] = minv[i];
+        l_r[lr] = first ? bi : r[i];
+        l_r0[lr] = first ? bi : r0[i];
+        l_p[lr] = first ? 0.0 : p[i];
+        l_v[lr] = first ? 0.0 : v[i];
+        l_x[lr] = first ? 0.0 : x[i];
+        d[0] += bi * bi;
+    });
+    bool alive = true;
+    if (first)
+    {
+        alive = ex.sum<1>(d);
+        if (alive) s = bicg_first_state(d[0], cuda_rule, tol, max_it);
+        if (s.done) iters = 0;
+    }
+    for (int k = 0; alive && k < iters; ++k)
+    {
+        double* const p_hat = ring + int64_t(3 * k) * stride;
+        double* const s_hat = p_hat + stride;
+        if (!cuda_rule && bicg_restart_due(s))
+        {
+            double* const xs = s_hat + stride;
+            each([&](int lr, int64_t i) { publish(xs + i, l_x[lr]); });
+            alive = ex.sum<0>(d);
+            if (!alive) break;
+            rows.template product<double, double>(g, first_row, false, xs, l_y, part);
+            d[0] = 0.0;
+            each([&](int lr, int64_t) {
+                double const ri = l_b[lr] - rows.result(g, l_y, part, lr);
+                l_r[lr] = ri;
+                l_r0[lr] = ri;
+                d[0] += ri * ri;
+            });
+            alive = ex.sum<1>(d);
+            if (!alive) break;
+            bicg_restarted(s, d[0]);
+        }
+        {
+            bool const plain = cuda_rule && s.it == 0;
+            double const beta = (s.rz / s.aux0) * (s.alpha / s.omega), omega = s.omega;
+            each([&](int lr, int64_t i) {
+                double const pi = plain ? l_r[lr] : l_r[lr] + beta * (l_p[lr] - omega * l_v[lr]);
+                l_p[lr] = pi;
+                publish(p_hat + i, l_m[lr] * pi);
+            });
+        }
+        alive = ex.sum<0>(d);
+        if (!alive) break;
+        rows.template product<double, double>(g, first_row, false, p_hat, l_y, part);
+        d[0] = 0.0;
+        each([&](int lr, int64_t) {
+            double const vi = rows.result(g, l_y, part, lr);
+            l_v[lr] = vi;
+            d[0] += l_r0[lr] * vi;
+        });
+        alive = ex.sum<1>(d);
+        if (!alive) break;
+        double const alpha = s.rz / d[0];
+        d[0] = 0.0;
+        each([&](int lr, int64_t i) {
+            double const si = l_r[lr] - alpha * l_v[lr];
+            l_r[lr] = si;
+            publish(s_hat + i, l_m[lr] * si);
+            d[0] += si * si;
+        });
+        alive = ex.sum<1>(d);
+        if (!alive) break;
+        s.alpha = alpha;
+        s.aux1 = sqrt(d[0]);
+        s.refine = cuda_rule && sqrt(d[0]) < tol ? 1 : 0;
+        if (s.refine)
+        {
+            each([&](int lr, int64_t) { l_x[lr] += alpha * (l_m[lr] * l_p[lr]); });
+            bicg_decide(s, 0.0, 0.0, 0.0, 0.0, cuda_rule, tol, max_it);
+            break;
+        }
+        rows.template product<double, double>(g, first_row, true, s_hat, l_y, part);
+        d[0] = d[1] = 0.0;
+        each([&](int lr, int64_t) {
+            double const ti = rows.result(g, l_y, part, lr);
+            if (!ROWS::kSliced || g.wps > 1) l_y[lr] = ti;
+            d[0] += ti * l_r[lr];
+            d[1] += ti * ti;
+        });
+        alive = ex.sum<2>(d);
+        if (!alive) break;
+        double const ts = d[0], tt = d[1];
+        double const omega = cuda_rule ? ts / tt : (tt > 0.0 ? ts / tt : 0.0);
+        d[0] = d[1] = 0.0;
+        each([&](int lr, int64_t) {
+            double const ph = l_m[lr] * l_p[lr], sh = l_m[lr] * l_r[lr];
+            if (cuda_rule)
+            {
+                // x = x + alpha p_hat + omega s_hat as two updates (the two cublasDaxpy calls)
+                double const xi = l_x[lr] + alpha * ph;
+                l_x[lr] = xi + omega * sh;
+            }
+            else
+                l_x[lr] += alpha * ph + omega * sh; // x += (alpha y + w z)
+            double const ri = l_r[lr] - omega * l_y[lr];
+            l_r[lr] = ri;
+            d[0] += l_r0[lr] * ri;
+            d[1] += ri * ri;
+        });
+        alive = ex.sum<2>(d);
+        if (!alive) break;
+        bicg_decide(s, ts, tt, d[0], d[1], cuda_rule, tol, max_it);
+        if (s.done) break;
+    }
+    if (alive)
+        each([&](int lr, int64_t i) {
+            x[i] = l_x[lr];
+            r[i] = l_r[lr];
+            r0[i] = l_r0[lr];
+            p[i] = l_p[lr];
+            v[i] = l_v[lr];
+        });
+    if (blockIdx.x == 0 && tid == 0)
+    {
+        if (!alive) s.done = KRYLOV_ABORTED;
+        *st = s;
+    }
+}
 } // namespace neon_amd

@@ -59,13 +59,22 @@ private:
     int count_;
 };
 
-// LDS residency: `most` 8-byte vectors of the block's rows if they fit, else `least` of them
-bool fit_lds(grid_shape& g, int64_t extra, int most, int most_elems, int least, int least_elems)
+// The vectors of a loop's recurrence: all of them in LDS, or the fewest that must be (0: all), and the
+// most rows per thread in either case
+struct vector_need
+{
+    int all, all_rows, least, least_rows;
+};
+constexpr vector_need kCgNeed{5, kGridElems<true>, 3, kGridElems<false>};
+constexpr vector_need kBicgNeed{kGridBicgVectors, 64, 0, 0};
+
+bool fit_lds(grid_shape& g, int64_t extra, vector_need need)
 {
     for (bool all : {true, false})
     {
-        int64_t const bytes = int64_t(g.rows) * 8 * (all ? most : least) + extra;
-        if (bytes > kGridLds || g.rows > kGridThreads * (all ? most_elems : least_elems)) continue;
+        if (!all && need.least == 0) break;
+        int64_t const bytes = int64_t(g.rows) * 8 * (all ? need.all : need.least) + extra;
+        if (bytes > kGridLds || g.rows > kGridThreads * (all ? need.all_rows : need.least_rows)) continue;
         g.all = all;
         g.lds = bytes;
         return true;
@@ -79,7 +88,8 @@ bool fit_lds(grid_shape& g, int64_t extra, int most, int most_elems, int least, 
 // itself waits for the longest slice.  Sharing a slice among wavefronts spreads few slices over all
 // compute units and evens out slices of unequal length; without need it only adds rounds (41 x 40 x
 // 38 cells, 1,050 slices: 14.4 us per product with one wavefront per slice, 15.1 with eight).
-bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_t most_items, int units)
+bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_t most_items, int units,
+                  vector_need need)
 {
     int const most = std::min(units, kGridMaxBlocks) / 8; // blocks per XCD
     if (most < 1 || per_xcd < 1) return false;
@@ -98,7 +108,7 @@ bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_
         double const cost = t.rounds * (2.0 + (wps == 1 ? most_items : mean / wps));
         int64_t const extra = (wps > 1 ? int64_t(t.rows) * wps * 8 : 0) + int64_t(t.rounds) * groups * 4;
         if (best > 0.0 && cost >= best) continue;
-        if (!fit_lds(t, extra, 5, kGridElems<true>, 3, kGridElems<false>)) continue;
+        if (!fit_lds(t, extra, need)) continue;
         best = cost;
         g = t;
     }
@@ -106,16 +116,16 @@ bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_
 }
 
 // Shape of a CSR grid: at least 64 rows per block
-bool shape_csr(grid_shape& g, int64_t n, int units)
+bool shape_csr(grid_shape& g, int64_t n, int units, vector_need need)
 {
     int64_t const most = std::min(units, kGridMaxBlocks);
     int64_t rows = std::max<int64_t>(64, (n + most - 1) / most);
     rows = (rows + 15) / 16 * 16;
-    if (rows > kGridThreads * kGridElems<false>) return false;
+    if (rows > 64 * kGridThreads) return false;
     g.n = n;
     g.rows = int32_t(rows);
     g.blocks = int32_t((n + rows - 1) / rows);
-    return fit_lds(g, kCsrChunk * 8 + 4 * (rows + 1), 5, kGridElems<true>, 3, kGridElems<false>);
+    return fit_lds(g, kCsrChunk * 8 + 4 * (rows + 1), need);
 }
 
 template <typename K>
@@ -136,6 +146,15 @@ sym_matrix sym_of(linear_operator const& A)
 sell_matrix sell_of(linear_operator const& A)
 {
     return sell_matrix{A.nodes, A.slices, A.sptr, A.snode, A.slane, A.scode, A.sexc, A.soff16, A.soff32};
+}
+
+bool shape_of(grid_shape& g, linear_operator const& A, int units, vector_need need)
+{
+    if (A.node_block && A.sym)
+        return shape_sliced(g, A.n, A.sym_slots / 8, 1.0 + A.sym_mean, 1 + A.sym_entries, units, need);
+    if (A.node_block && A.sell)
+        return shape_sliced(g, A.n, (A.slices + 7) / 8, A.sell_mean, A.sell_steps, units, need);
+    return !A.node_block && shape_csr(g, A.n, units, need);
 }
 } // namespace
 
@@ -202,14 +221,7 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
     grid_begin();
     if (!grid_units_ || A.blocks_override > 0) return false;
     grid_shape g;
-    bool ok = false;
-    if (A.node_block && A.sym)
-        ok = shape_sliced(g, A.n, A.sym_slots / 8, 1.0 + A.sym_mean, 1 + A.sym_entries, grid_units_);
-    else if (A.node_block && A.sell)
-        ok = shape_sliced(g, A.n, (A.slices + 7) / 8, A.sell_mean, A.sell_steps, grid_units_);
-    else if (!A.node_block)
-        ok = shape_csr(g, A.n, grid_units_);
-    if (!ok) return false;
+    if (!shape_of(g, A, grid_units_, kCgNeed)) return false;
 
     int64_t const n = A.n;
     int64_t const stride = (n + 31) / 32 * 32; // whole 128-byte lines
@@ -280,6 +292,69 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
     if (!done) return false;
     out = finish_solve(*host_state_, criterion);
     out.spmv = out.iterations + (criterion == NEON_STOP_RELATIVE && host_state_->done == KRYLOV_CONVERGED ? 1 : 0);
+    return true;
+}
+
+bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, double* x, const double* minv,
+                                    int criterion, double tol, int32_t max_it, const krylov_work* work,
+                                    solve_result& out)
+{
+    if (prof && prof->enabled) return false;
+    grid_begin();
+    if (!grid_units_ || A.blocks_override > 0) return false;
+    grid_shape g;
+    if (!shape_of(g, A, grid_units_, kBicgNeed)) return false;
+    int64_t const n = A.n;
+    int64_t const stride = (n + 31) / 32 * 32; // whole 128-byte lines
+    double *r, *r0, *p, *v, *ring;
+    int64_t buffers;
+    if (work)
+    {
+        r = work->r, r0 = work->r0, p = work->p, v = work->v;
+        ring = work->bicg_ring;
+        buffers = work->bicg_ring_size / stride;
+    }
+    else
+    {
+        grid_bicg_.reserve(4 * stride);
+        r = grid_bicg_.data(), r0 = r + stride, p = r0 + stride, v = p + stride;
+        buffers = std::clamp<int64_t>(kGridRing / stride, 12, 96);
+        grid_ring_.reserve(buffers * stride);
+        ring = grid_ring_.data();
+    }
+    int const iters = int(std::min<int64_t>(buffers / 3, 32));
+    if (iters < 1) return false;
+    int const cuda_rule = criterion == NEON_STOP_ABSOLUTE_PRECONDITIONED ? 1 : 0;
+    krylov_state* st = state_.data() + 2;
+    unit_hold const hold(grid_device_, g.blocks, grid_units_);
+    auto launch = [&](auto rows) {
+        auto kernel = bicg_grid_kernel<decltype(rows)>;
+        allow_lds(kernel, g.lds);
+        return grid_run([&, kernel](bool first) {
+            kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, b, x, r, r0, p, v, minv, st,
+                                                                  grid_next(uint32_t(7 * iters + 1)), first ? 1 : 0,
+                                                                  iters, cuda_rule, tol, max_it);
+        });
+    };
+    bool done = false;
+    if (A.sym)
+        done = launch(grid_sliced<grid_sym<double>>{{sym_of(A), A.s64}});
+    else if (A.sell)
+    {
+        using lay = grid_sell<double>;
+        lay const l{sell_of(A), A.s64};
+        int const items = (A.sell_steps + g.wps - 1) / g.wps;
+        if (g.rounds == 1 && g.wps == 8 && items <= 4)
+            done = launch(grid_kept<lay, 4, 8>{{l}, {}});
+        else if (g.rounds == 1 && g.wps == 4 && items <= 8)
+            done = launch(grid_kept<lay, 8, 4>{{l}, {}});
+        else
+            done = launch(grid_sliced<lay>{l});
+    }
+    else
+        done = launch(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}});
+    if (!done) return false;
+    out = finish_bicg(*host_state_, criterion);
     return true;
 }
 } // namespace neon_amd

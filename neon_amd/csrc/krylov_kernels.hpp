@@ -942,42 +942,7 @@ __global__ __launch_bounds__(kBlock) void bicg_finish_kernel(const double* __res
     }
     if (threadIdx.x != 0) return;
     krylov_state s = *st;
-    int32_t const k = s.it + 1;
-    if (cuda_rule)
-    {
-        if (s.refine)
-        {
-            // ||s|| < tol: x += alpha p_hat, residual = ||s||^2, leave the loop
-            s.rz = s.aux1 * s.aux1;
-            s.done = k >= max_it ? KRYLOV_LIMIT : KRYLOV_CONVERGED;
-        }
-        else
-        {
-            s.omega = ts / tt;
-            s.aux0 = s.rz;
-            s.rz = r0r;
-            if (s.omega == 0.0) // is_approx(omega, 0.0): an exact zero
-                s.done = KRYLOV_BREAKDOWN;
-            else if (!(sqrt(s.rz) > tol) || k >= max_it)
-                s.done = k >= max_it ? KRYLOV_LIMIT : KRYLOV_CONVERGED;
-            if (!isfinite(s.rz) && s.done != KRYLOV_BREAKDOWN) s.done = KRYLOV_NONFINITE;
-        }
-        s.rr = rr;
-    }
-    else
-    {
-        s.omega = tt > 0.0 ? ts / tt : 0.0;
-        s.rr = rr;
-        s.aux0 = s.rz; // rho_old for the next iteration
-        s.rz = r0r;    // r0 . r, the next iteration's rho unless it restarts
-        if (!(rr > s.threshold))
-            s.done = KRYLOV_CONVERGED;
-        else if (k >= max_it)
-            s.done = KRYLOV_LIMIT;
-        if (!isfinite(rr)) s.done = KRYLOV_NONFINITE;
-    }
-    s.it = k;
-    s.refine = 0;
+    bicg_decide(s, ts, tt, r0r, rr, cuda_rule, tol, max_it);
     *st = s;
 }
 
@@ -986,8 +951,7 @@ __global__ __launch_bounds__(kBlock) void bicg_finish_kernel(const double* __res
 __global__ __launch_bounds__(kBlock) void bicg_restart_test_kernel(krylov_state* __restrict__ st)
 {
     if (threadIdx.x != 0 || st->done) return;
-    double const eps2 = DBL_EPSILON * DBL_EPSILON;
-    st->refine = fabs(st->rz) < eps2 * st->aux1 ? 1 : 0;
+    st->refine = bicg_restart_due(*st) ? 1 : 0;
 }
 
 // Eigen rule, restart (gated on refine): r0 = r (the fresh residual), partials of r.r
@@ -1016,10 +980,7 @@ __global__ __launch_bounds__(kBlock) void bicg_restart_finish_kernel(const doubl
     if (st->done || !st->refine) return;
     double const rr = reduce_partials<kBlock>(part_rr, npart);
     if (threadIdx.x != 0) return;
-    st->rz = rr;
-    st->aux1 = rr;
-    if (st->restarts++ == 0) st->it = 0;
-    st->refine = 0;
+    bicg_restarted(*st, rr);
 }
 
 // ------------------------------------------------------- generic vector kernels

@@ -337,4 +337,93 @@ __device__ inline double cg_decide(krylov_state& s, double rr, double rz, int cr
     s.done = done;
     return beta;
 }
+
+// The state a BiCGSTAB solve starts from (x = 0, r = r0 = b), given b.b
+__host__ __device__ inline krylov_state bicg_first_state(double bb, int cuda_rule, double tol, int max_it)
+{
+    krylov_state s{};
+    s.rz = bb; // r0 . r = b . b
+    s.rr = bb;
+    s.rhs2 = bb;
+    s.aux0 = 1.0; // Eigen's rho_old, alpha, omega start at 1
+    s.alpha = 1.0;
+    s.omega = 1.0;
+    s.aux1 = bb; // Eigen's |r0|^2
+    if (cuda_rule)
+    {
+        s.aux0 = 0.0;
+        s.alpha = s.omega = 0.0;
+        if (!(sqrt(bb) > tol))
+            s.done = KRYLOV_CONVERGED;
+        else if (max_it <= 0)
+            s.done = KRYLOV_LIMIT;
+    }
+    else
+    {
+        s.threshold = tol * tol * bb;
+        if (bb == 0.0 || !(bb > s.threshold))
+            s.done = KRYLOV_CONVERGED;
+        else if (max_it <= 0)
+            s.done = KRYLOV_LIMIT;
+    }
+    if (!(fabs(bb) <= DBL_MAX)) s.done = KRYLOV_NONFINITE;
+    return s;
+}
+
+// The Eigen rule's restart test |rho| < eps^2 |r0|^2 and the scalars after a restart with |r|^2 = rr
+// (the first one resets the iteration count)
+__device__ inline bool bicg_restart_due(krylov_state const& s)
+{
+    return fabs(s.rz) < DBL_EPSILON * DBL_EPSILON * s.aux1;
+}
+__device__ inline void bicg_restarted(krylov_state& s, double rr)
+{
+    s.rz = rr;
+    s.aux1 = rr;
+    if (s.restarts++ == 0) s.it = 0;
+    s.refine = 0;
+}
+
+// End of a BiCGSTAB iteration: s <- its scalars, count and status (s.refine: the CUDA rule's early
+// exit; ts, tt, r0r and rr are then unused)
+__device__ inline void bicg_decide(krylov_state& s, double ts, double tt, double r0r, double rr, int cuda_rule,
+                                   double tol, int max_it)
+{
+    int32_t const k = s.it + 1;
+    if (cuda_rule)
+    {
+        if (s.refine)
+        {
+            // ||s|| < tol: x += alpha p_hat, residual = ||s||^2, leave the loop
+            s.rz = s.aux1 * s.aux1;
+            s.done = k >= max_it ? KRYLOV_LIMIT : KRYLOV_CONVERGED;
+        }
+        else
+        {
+            s.omega = ts / tt;
+            s.aux0 = s.rz;
+            s.rz = r0r;
+            if (s.omega == 0.0) // is_approx(omega, 0.0): an exact zero
+                s.done = KRYLOV_BREAKDOWN;
+            else if (!(sqrt(s.rz) > tol) || k >= max_it)
+                s.done = k >= max_it ? KRYLOV_LIMIT : KRYLOV_CONVERGED;
+            if (!isfinite(s.rz) && s.done != KRYLOV_BREAKDOWN) s.done = KRYLOV_NONFINITE;
+        }
+        s.rr = rr;
+    }
+    else
+    {
+        s.omega = tt > 0.0 ? ts / tt : 0.0;
+        s.rr = rr;
+        s.aux0 = s.rz; // rho_old for the next iteration
+        s.rz = r0r;    // r0 . r, the next iteration's rho unless it restarts
+        if (!(rr > s.threshold))
+            s.done = KRYLOV_CONVERGED;
+        else if (k >= max_it)
+            s.done = KRYLOV_LIMIT;
+        if (!isfinite(rr)) s.done = KRYLOV_NONFINITE;
+    }
+    s.it = k;
+    s.refine = 0;
+}
 } // namespace neon_amd

@@ -206,3 +206,84 @@ def test_two_contexts_share_the_gpu():
     for k in range(2):
         assert results[k][3] <= 1.1e-10
         assert np.array_equal(results[k][0], results[k][1]) and np.array_equal(results[k][0], results[k][2])
+
+
+def _unsymmetric(n, per_row, seed):
+    A, b = _spd(n, per_row, seed)
+    rng = np.random.default_rng(seed + 1)
+    A = A.copy()
+    A.data *= rng.uniform(0.5, 1.0, len(A.data))
+    return (A + sp.diags(np.abs(A).sum(axis=1).A1 + 1.0)).tocsr(), b
+
+
+# BiCGSTAB follows roundoff closely (test_bicgstab_host_csr_parity): counts within 15 % and 3; its
+# recurrence residual drifts from the true one by eps |A| |x| per iteration times the largest
+# residual on the way, some orders below 1e-10 |b| on these diagonally dominant systems
+@pytest.mark.parametrize("n,per_row", [(1, 1), (63, 4), (65, 5), (900, 60), (20000, 30), (262143, 9), (700000, 5)])
+def test_bicgstab_on_host_csr(ctx, n, per_row):
+    print(n, per_row, flush=True)
+    A, b = _unsymmetric(n, per_row, n)
+    grid, launches = _both(ctx, lambda: _solve_csr(ctx, neon_amd.biconjugate_gradient_stabilised_hip, A, b))
+    for x, its, _ in (grid, launches):
+        assert np.linalg.norm(b - A @ x) <= 2e-10 * np.linalg.norm(b)
+    assert abs(grid[1] - launches[1]) <= 3 + 0.15 * launches[1], (grid[1], launches[1])
+
+
+# the unsymmetric tangent on the full copy with eight and four wavefronts per slice, its share of the
+# matrix in registers; several rounds; one wavefront per slice; and a symmetric copy
+@pytest.mark.parametrize("dims,model", [((3, 4, 3), "damage"), ((12, 11, 13), "damage"), ((30, 29, 31), "damage"),
+                                        ((36, 35, 37), "damage"), ((45, 44, 43), "damage"), ((20, 21, 19), "neohooke")])
+def test_bicgstab_on_the_mesh_tangent(ctx, dims, model):
+    print(dims, model, flush=True)
+    p = problems.block_rollers(max(dims), dims=dims)
+    if model == "damage":
+        q = problems.damage_cube(1)
+        params = np.repeat(q.params[:1], p.n_elem, axis=0)
+        mg = neon_amd.DeviceMesh(p.X, p.conn, params, model=neon_amd.MODEL_J2_DAMAGE, context=ctx,
+                                 damage=problems.DAMAGE_CONSTANTS)
+    else:
+        mg = neon_amd.DeviceMesh(p.X, p.conn, p.params, context=ctx)
+        mg.update_internal_variables()
+    mg.assemble()
+    b = np.random.default_rng(12).standard_normal(mg.n_dofs)
+    mg.enforce_dirichlet(p.fixed_dofs(), b)
+    A = _matrix(mg)
+    # the right-hand side of a solution of order one
+    b = A @ b
+    grid, launches = _both(ctx, lambda: mg.solve(b, solver=neon_amd.SOLVER_BICGSTAB, tol=1e-10))
+    for x, its, _ in (grid, launches):
+        assert np.linalg.norm(b - A @ x) <= 2e-10 * np.linalg.norm(b)
+    assert abs(grid[1] - launches[1]) <= 3 + 0.15 * launches[1], (grid[1], launches[1])
+
+
+@pytest.mark.parametrize("criterion", [neon_amd.STOP_RELATIVE, neon_amd.STOP_ABSOLUTE_PRECONDITIONED])
+def test_bicgstab_ends(ctx, criterion):
+    """The CUDA rule's early exit (an identity matrix), a zero right-hand side, the iteration limit
+    inside and past a launch, and values that are not finite end as they do by launches."""
+    cls = neon_amd.biconjugate_gradient_stabilised_hip
+
+    def outcome(A, b, tol, limit):
+        got = []
+        for timed in (False, True):
+            s = cls(tol, limit, criterion=criterion, context=ctx)
+            x = np.zeros(len(b))
+            ctx.profile(timed)
+            try:
+                s.solve(A, x, b)
+                code = 0
+            except neon_amd.computational_error as e:
+                code = e.code
+            finally:
+                ctx.profile(False)
+            got.append((code, s.iterations))
+        assert got[0] == got[1], got
+        return got[0]
+
+    ident = sp.identity(500, format="csr")
+    b = np.linspace(1.0, 2.0, 500)
+    assert outcome(ident, b, 1e-10, 100)[0] in (0, _capi.NEON_BREAKDOWN, _capi.NEON_NAN_OR_INF)
+    assert outcome(ident, np.zeros(500), 1e-10, 100) == (0, 0)
+    A, b = _unsymmetric(2000, 12, 4)
+    assert outcome(A, b, 1e-30, 3) == (_capi.NEON_NONCONVERGED, 3)
+    b[5] = np.nan
+    assert outcome(A, b, 1e-10, 100)[0] == _capi.NEON_NAN_OR_INF
