@@ -1136,11 +1136,22 @@ int device_mesh::update_internal_variables(const double* u_dev, double dt)
     switch (model_ & 0xff)
     {
     case NEON_MODEL_J2_DAMAGE:
-        damage_update_kernel<<<grid_for(Q), kBlock, 0, s_>>>(
-            E_, conn_.data(), X_.data(), u_dev, prm, st,
-            damage_state{dmg_state_.data(), dmg_state_.data() + 6 * Q, dmg_state_.data() + 7 * Q},
-            damage_constants{damage_[0], damage_[1], damage_[2], damage_[3], damage_[4], damage_[5]}, dt,
-            status_.data());
+    {
+        damage_state const ds{dmg_state_.data(), dmg_state_.data() + 6 * Q, dmg_state_.data() + 7 * Q};
+        damage_constants const dc{damage_[0], damage_[1], damage_[2], damage_[3], damage_[4], damage_[5]};
+        yield_.reserve(size_t(Q) + 1);
+        NEON_CHECK_HIP(hipMemsetAsync(yield_.data(), 0, sizeof(int32_t), s_));
+        damage_predict_kernel<<<grid_for(Q), kBlock, 0, s_>>>(E_, conn_.data(), X_.data(), u_dev, prm, st, ds, dc,
+                                                              status_.data(), yield_.data());
+        NEON_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(damage_return_kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           int(sizeof(damage_detail::damage_lds))));
+        // one workgroup fills a compute unit's LDS: two rounds of them at most, striding over the list
+        int const blocks = int(std::min<int64_t>((Q + damage_detail::kDamagePoints - 1) / damage_detail::kDamagePoints, 512));
+        damage_return_kernel<<<blocks, 256, sizeof(damage_detail::damage_lds), s_>>>(
+            conn_.data(), X_.data(), u_dev, prm, st, ds, dc, std::pow(dc.sp, -dc.np), std::pow(dc.sd, -dc.nd), dt,
+            status_.data(), yield_.data());
+    }
         break;
     case NEON_MODEL_NEOHOOKE: NEON_UPDATE(NEON_MODEL_NEOHOOKE); break;
     case NEON_MODEL_J2: NEON_UPDATE(NEON_MODEL_J2); break;

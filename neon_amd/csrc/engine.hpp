@@ -444,6 +444,7 @@ private:
     // J2 damage: back stress 6, damage 1, energy release rate 1 per QP (SoA) and the committed
     // back stress and damage; the material's constants (C, gamma, s_p, n_p, s_d, n_d)
     device_array<double> dmg_state_, dmg_state_old_;
+    device_array<int32_t> yield_; // an update's yielding points: their count, then their numbers
     double damage_[6] = {1.0, 1.0, 1.0, 1.0, 1.0, 1.0};
     device_array<uint32_t> status_;
     std::vector<std::unique_ptr<device_array<double>>> traj_u_, traj_ep_, traj_eb_;

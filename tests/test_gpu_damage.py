@@ -100,3 +100,26 @@ def test_newton_cube_parity(ctx, n, top):
     dg, dr = mg.damage_state(), mr.damage_state()
     _close(dg["damage"], dr["damage"], 1e-8, "damage")
     assert (dr["damage"] > 0).all()
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (3, 3, 1), (3, 3, 3)])
+def test_return_map_groups_parity(ctx, dims):
+    """The return map handles 64 yielding points per workgroup, taken from a list: one element (8
+    points), exactly one group, one point group more, and several, some of the points elastic (the
+    pull grows from nothing along x), against the oracle (tolerances of the sequence test)."""
+    print(dims, flush=True)
+    X, conn, _ = problems.box_mesh(*dims, L=(1.0, 1.0, 1.0), jitter=0.1)
+    params = np.repeat(problems.damage_cube(1).params[:1], len(conn), axis=0)
+    mg = neon_amd.DeviceMesh(X, conn, params, model=neon_amd.MODEL_J2_DAMAGE, context=ctx, damage=CONST)
+    mr = orc.Model(X, conn, params, model=orc.MODEL_J2_DAMAGE)
+    mr.set_damage(CONST)
+    u = np.zeros_like(X)
+    u[:, 2] = 0.0025 * X[:, 2] * X[:, 0]
+    u[:, 0] = -0.0007 * X[:, 0] * X[:, 2]
+    u = u.reshape(-1)
+    mg.set_displacement(u)
+    mg.update_internal_variables(1e-3)
+    assert mr.update(u, 1e-3) == orc.OK
+    sg, sr = mg.qp_state(), mr.qp_state()
+    for key in ("sigma", "D", "eps_p", "ebar", "vm"):
+        _close(sg[key], sr[key], 1e-9, key)
