@@ -217,6 +217,7 @@ int neon_krylov_solve_csr(neon_context* ctx, int solver, int criterion, int prec
         linear_operator A;
         A.n = n;
         A.node_block = false;
+        A.nnz = nnz;
         A.rp = rp.data();
         A.ci = ci.data();
         A.lanes_per_row = lanes_for(double(nnz) / n);
@@ -273,6 +274,7 @@ int neon_krylov_solve_csr_noalloc(neon_context* ctx, int solver, int criterion, 
         linear_operator A;
         A.n = n;
         A.node_block = false;
+        A.nnz = nnz;
         A.rp = row_ptr;
         A.ci = col;
         A.lanes_per_row = lanes_for(double(nnz) / n);

@@ -104,6 +104,7 @@ struct sym_matrix; // krylov_kernels.hpp
 struct linear_operator
 {
     int64_t n = 0;
+    int64_t nnz = 0; // generic CSR layout only
     bool node_block = false;
     // node-block layout
     int32_t nodes = 0;

@@ -796,7 +796,10 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_kernel(ROWS rows, grid_s
     }
     for (int k = 0; alive && k < iters; ++k)
     {
-        rows.template product<double, double>(g, first_row, (k & 1) != 0, ring + int64_t(k) * stride, l_z, part);
+        if (!ROWS::kSliced && g.blocks == 1) // local rows are the system's: p is gathered from LDS
+            rows.template product<double, double>(g, first_row, false, static_cast<const double*>(l_p), l_z, part);
+        else
+            rows.template product<double, double>(g, first_row, (k & 1) != 0, ring + int64_t(k) * stride, l_z, part);
         v[0] = 0.0;
         int t = here(tid);
         double mi[ALL ? 1 : EL], xi[ALL ? 1 : EL];
@@ -852,7 +855,7 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_kernel(ROWS rows, grid_s
             double const old = l_p[lr];
             double const pi = l_z[lr] + beta * old;
             l_p[lr] = pi;
-            if (!s.done) publish(next + i, pi);
+            if (!s.done && (ROWS::kSliced || g.blocks > 1 || last)) publish(next + i, pi);
             if constexpr (ALL)
                 l_x[lr] += alpha * old;
             else
