@@ -225,6 +225,16 @@ void kernel_profiler::read(int cls, bool reset, int64_t* count, double* ms)
 }
 
 // ================================================================== engine
+csr_space::csr_space()
+{
+    NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&stage), kCsrStage));
+}
+
+csr_space::~csr_space()
+{
+    if (stage) (void)hipHostFree(stage);
+}
+
 krylov_engine::krylov_engine(hipStream_t s) : s_(s)
 {
     // partials, then their total (totals_kernel)

@@ -182,9 +182,27 @@ constexpr int64_t kGridRing = int64_t(1) << 23;
 solve_result finish_solve(const krylov_state& s, int criterion);
 solve_result finish_bicg(const krylov_state& s, int criterion);
 
+// Device memory and a pinned buffer that the host-CSR solves of one context keep from call to call
+// (a program solves many systems of one size; a small solve spent half its time on seven
+// allocations and five pageable copies).  At most kCsrKept bytes stay after a call; the context
+// frees the rest with it.
+constexpr size_t kCsrKept = size_t(256) << 20;
+constexpr size_t kCsrStage = size_t(256) << 10; // pinned
+struct csr_space
+{
+    device_array<unsigned char> dev;
+    unsigned char* stage = nullptr;
+    csr_space();
+    ~csr_space();
+    csr_space(csr_space const&) = delete;
+    csr_space& operator=(csr_space const&) = delete;
+};
+
 class krylov_engine
 {
 public:
+    csr_space csr;
+
     explicit krylov_engine(hipStream_t s);
     ~krylov_engine();
 
