@@ -378,27 +378,39 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
     double* part_rz = part_[2].data();
     krylov_state* st = state_.data();
 
-    cg_init_kernel<<<nb, kBlock, 0, s_>>>(n, x, r, p, b, minv, part_rr, part_rz);
-    cg_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, criterion, tol, max_it);
-    NEON_CHECK_HIP(hipGetLastError());
-
+    // with the vector part of an iteration in one launch, and again without if that gave up
     int64_t launched = 0;
-    linear_operator Ak = A; // its products alternate in order
-    run_batches(st, launched, [&] {
-        for (int k = 0; k < poll_every; ++k, ++launched)
-        {
-            krylov_state* cur = st + (launched & 1);
-            krylov_state* nxt = st + ((launched + 1) & 1);
-            int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP64) : -1;
-            Ak.back = int(launched & 1);
-            Ak.apply64(s_, p, Ap, part_pAp, cur);
-            if (prof) prof->end(s_, tok);
-            totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
-            cg_update_xr_kernel<<<nb, kBlock, 0, s_>>>(n, r, Ap, minv, part_pAp, -1, cur, part_rr, part_rz);
-            cg_update_p_kernel<<<nb, kBlock, 0, s_>>>(n, p, x, r, minv, part_pAp, part_rr, part_rz, nb, cur, nxt,
-                                                       criterion, tol, max_it);
-        }
-    });
+    for (int vb = vector_blocks(n, 2);; vb = 0)
+    {
+        cg_init_kernel<<<nb, kBlock, 0, s_>>>(n, x, r, p, b, minv, part_rr, part_rz);
+        cg_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, criterion, tol, max_it);
+        NEON_CHECK_HIP(hipGetLastError());
+        auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        launched = 0;
+        linear_operator Ak = A; // its products alternate in order
+        run_batches(st, launched, [&] {
+            for (int k = 0; k < poll_every; ++k, ++launched)
+            {
+                krylov_state* cur = st + (launched & 1);
+                krylov_state* nxt = st + ((launched + 1) & 1);
+                int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP64) : -1;
+                Ak.back = int(launched & 1);
+                Ak.apply64(s_, p, Ap, part_pAp, cur);
+                if (prof) prof->end(s_, tok);
+                if (vb)
+                {
+                    cg_vector(vb, n, r, Ap, minv, x, p, part_pAp, ns, cur, nxt, criterion, tol, max_it);
+                    continue;
+                }
+                totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
+                cg_update_xr_kernel<<<nb, kBlock, 0, s_>>>(n, r, Ap, minv, part_pAp, -1, cur, part_rr, part_rz);
+                cg_update_p_kernel<<<nb, kBlock, 0, s_>>>(n, p, x, r, minv, part_pAp, part_rr, part_rz, nb, cur, nxt,
+                                                           criterion, tol, max_it);
+            }
+        });
+        if (!vb || !vector_gave_up()) break;
+        if (prof) prof->discard();
+    }
     res = finish_solve(*host_state_, criterion);
     // SpMV launches that did work: Eigen's rule counts the converging iteration's SpMV
     // outside `iterations`; the CUDA rule counts every iteration.
@@ -596,61 +608,75 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     // r = b - K x64 use A, the unscaled FP32 values, so convergence is judged on K as without it
     bool const scaled = minv64_scaled != nullptr;
     linear_operator Ak = scaled ? *scaled_op : A; // its products alternate in order
-    if (scaled)
-        mixed_init_scaled_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv64_scaled, part_rr, part_rz);
-    else
-        mixed_init_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv, part_rr, part_rz);
-    mixed_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, tol, max_it);
-    NEON_CHECK_HIP(hipGetLastError());
-    // the gated true-residual product is a no-op in all but a few of its launches: a grid of at
-    // most 2,048 workgroups striding over the slices keeps those launches short
-    linear_operator Ar = A;
-    if (Ar.node_block && (Ar.sell || Ar.sym)) Ar.blocks_override = 2048;
+    // the iterations without a decision with their vector part in one launch (scaled system), and all
+    // again without if that gave up
     int64_t launched = 0;
-    run_batches(st, launched, [&] {
-        for (int k = 0; k < poll_every; ++k, ++launched)
-        {
-            krylov_state* cur = st + (launched & 1);
-            krylov_state* nxt = st + ((launched + 1) & 1);
-            int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP32) : -1;
-            Ak.back = int(launched & 1);
-            Ak.apply32(s_, p32, Ap32, part_pAp, cur);
-            if (prof) prof->end(s_, tok);
-            totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
-            // the reliable-update / true-residual convergence test runs every refine_every
-            // iterations
-            int const decided = (launched + 1) % refine_every == 0 ? 1 : 0;
-            if (!scaled)
-                mixed_update_xr_kernel<false, true>
-                    <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, minv, part_pAp, -1, cur, part_rr, part_rz);
-            else if (decided)
-                mixed_update_xr_kernel<true, true>
-                    <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, minv, part_pAp, -1, cur, part_rr, part_rz);
-            else
-                mixed_update_xr_kernel<true, false>
-                    <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, nullptr, part_pAp, -1, cur, nullptr, part_rz);
-            if (decided)
+    for (int vb = scaled ? vector_blocks(n, 4) : 0;; vb = 0)
+    {
+        auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        if (scaled)
+            mixed_init_scaled_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv64_scaled, part_rr, part_rz);
+        else
+            mixed_init_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv, part_rr, part_rz);
+        mixed_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, tol, max_it);
+        NEON_CHECK_HIP(hipGetLastError());
+        // the gated true-residual product is a no-op in all but a few of its launches: a grid of at
+        // most 2,048 workgroups striding over the slices keeps those launches short
+        linear_operator Ar = A;
+        if (Ar.node_block && (Ar.sell || Ar.sym)) Ar.blocks_override = 2048;
+        launched = 0;
+        run_batches(st, launched, [&] {
+            for (int k = 0; k < poll_every; ++k, ++launched)
             {
-                mixed_decide_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, cur, reliable_delta);
-                mixed_fold_kernel<<<nb, kBlock, 0, s_>>>(n, x, x32, p32, part_pAp, cur, 0, minv64_scaled);
-                Ar.residual64(s_, b, x, r64, cur, 1);
-                if (scaled)
-                    mixed_refresh_kernel<true>
-                        <<<nb, kBlock, 0, s_>>>(n, r64, r32, minv, minv64_scaled, cur, part_rr_t, part_rz_t);
+                krylov_state* cur = st + (launched & 1);
+                krylov_state* nxt = st + ((launched + 1) & 1);
+                int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP32) : -1;
+                Ak.back = int(launched & 1);
+                Ak.apply32(s_, p32, Ap32, part_pAp, cur);
+                if (prof) prof->end(s_, tok);
+                // the reliable-update / true-residual convergence test runs every refine_every
+                // iterations
+                int const decided = (launched + 1) % refine_every == 0 ? 1 : 0;
+                if (vb && !decided)
+                {
+                    mixed_vector(vb, n, r32, Ap32, x32, p32, part_pAp, ns, cur, nxt, max_it);
+                    continue;
+                }
+                totals_kernel<<<1, 1024, 0, s_>>>(part_pAp, nullptr, ns, cur);
+                if (!scaled)
+                    mixed_update_xr_kernel<false, true>
+                        <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, minv, part_pAp, -1, cur, part_rr, part_rz);
+                else if (decided)
+                    mixed_update_xr_kernel<true, true>
+                        <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, minv, part_pAp, -1, cur, part_rr, part_rz);
                 else
-                    mixed_refresh_kernel<false>
-                        <<<nb, kBlock, 0, s_>>>(n, r64, r32, minv, nullptr, cur, part_rr_t, part_rz_t);
+                    mixed_update_xr_kernel<true, false>
+                        <<<nb, kBlock, 0, s_>>>(n, r32, Ap32, nullptr, part_pAp, -1, cur, nullptr, part_rz);
+                if (decided)
+                {
+                    mixed_decide_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, cur, reliable_delta);
+                    mixed_fold_kernel<<<nb, kBlock, 0, s_>>>(n, x, x32, p32, part_pAp, cur, 0, minv64_scaled);
+                    Ar.residual64(s_, b, x, r64, cur, 1);
+                    if (scaled)
+                        mixed_refresh_kernel<true>
+                            <<<nb, kBlock, 0, s_>>>(n, r64, r32, minv, minv64_scaled, cur, part_rr_t, part_rz_t);
+                    else
+                        mixed_refresh_kernel<false>
+                            <<<nb, kBlock, 0, s_>>>(n, r64, r32, minv, nullptr, cur, part_rr_t, part_rz_t);
+                }
+                if (scaled)
+                    mixed_update_p_kernel<true><<<nb, kBlock, 0, s_>>>(n, p32, x32, r32, nullptr, part_pAp, part_rr_t,
+                                                                       part_rz_t, part_rr, part_rz, nb, nb, decided, cur,
+                                                                       nxt, max_it);
+                else
+                    mixed_update_p_kernel<false><<<nb, kBlock, 0, s_>>>(n, p32, x32, r32, minv, part_pAp, part_rr_t,
+                                                                        part_rz_t, part_rr, part_rz, nb, nb, decided, cur,
+                                                                        nxt, max_it);
             }
-            if (scaled)
-                mixed_update_p_kernel<true><<<nb, kBlock, 0, s_>>>(n, p32, x32, r32, nullptr, part_pAp, part_rr_t,
-                                                                   part_rz_t, part_rr, part_rz, nb, nb, decided, cur,
-                                                                   nxt, max_it);
-            else
-                mixed_update_p_kernel<false><<<nb, kBlock, 0, s_>>>(n, p32, x32, r32, minv, part_pAp, part_rr_t,
-                                                                    part_rz_t, part_rr, part_rz, nb, nb, decided, cur,
-                                                                    nxt, max_it);
-        }
-    });
+        });
+        if (!vb || !vector_gave_up()) break;
+        if (prof) prof->discard();
+    }
     // fold whatever the recurrence holds since the last reliable update
     mixed_fold_kernel<<<nb, kBlock, 0, s_>>>(n, x, x32, p32, part_pAp, st + (launched & 1), 1, minv64_scaled);
     NEON_CHECK_HIP(hipGetLastError());

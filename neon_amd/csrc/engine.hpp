@@ -198,6 +198,9 @@ struct csr_space
     csr_space& operator=(csr_space const&) = delete;
 };
 
+class unit_hold; // grid_krylov.hip: compute units held for a resident grid
+std::shared_ptr<unit_hold> hold_units(int device, int count, int units);
+
 class krylov_engine
 {
 public:
@@ -273,6 +276,16 @@ private:
                    int32_t max_it, const krylov_work* work, solve_result& out);
     bool bicgstab64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion,
                          double tol, int32_t max_it, const krylov_work* work, solve_result& out);
+    // an iteration's vector part in one launch (vector_iteration): the workgroups for n entries (0:
+    // not available) and the launches; after a loop with them, whether one gave up (the loop then
+    // runs again without them)
+    int vector_blocks(int64_t n, int width);
+    void cg_vector(int blocks, int64_t n, double* r, const double* Ap, const double* minv, double* x, double* p,
+                   const double* part, int npart, const krylov_state* st, krylov_state* next, int criterion, double tol,
+                   int32_t max_it);
+    void mixed_vector(int blocks, int64_t n, float* r, const float* Ap, float* x, float* p, const double* part,
+                      int npart, const krylov_state* st, krylov_state* next, int32_t max_it);
+    bool vector_gave_up();
     void grid_begin();
     void grid_clear();
     grid_link grid_next(uint32_t exchanges);

@@ -121,13 +121,15 @@ __device__ inline void load_words(const uint64_t* p, word2 (&q)[NV])
                      : "memory");
 }
 
-// The exchange of one grid launch.  Every workgroup calls the same sequence of exchanges.
+// The exchange of one grid launch by workgroups of WAVES wavefronts.  Every workgroup calls the same
+// sequence of exchanges.
+template <int WAVES = kGridWaves>
 struct grid_exchange
 {
     grid_link link;
     int blocks;
-    double (*own)[2][kGridWaves]; // LDS [2 parities]: the wavefronts' sums
-    double (*all)[2][kGridWaves]; // LDS [2 parities]: the sums of the slots each wavefront read
+    double (*own)[2][WAVES]; // LDS [2 parities]: the wavefronts' sums
+    double (*all)[2][WAVES]; // LDS [2 parities]: the sums of the slots each wavefront read
     int* bad;                     // LDS
 
     // v[k] <- the sum over the grid, in a fixed order, for the values given by every thread; also
@@ -159,7 +161,7 @@ struct grid_exchange
             {
                 t[k] = 0.0;
 #pragma unroll
-                for (int w = 0; w < kGridWaves; ++w) t[k] += own[par][k][w];
+                for (int w = 0; w < WAVES; ++w) t[k] += own[par][k][w];
             }
         }
         if (blocks == 1)
@@ -758,7 +760,7 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_kernel(ROWS rows, grid_s
         reinterpret_cast<int32_t*>(part + (!ROWS::kSliced ? kCsrChunk : g.wps > 1 ? g.rows * g.wps : 0));
     rows.begin(g, first_row);
     __syncthreads();
-    grid_exchange ex{link, g.blocks, own, all, &bad};
+    grid_exchange<> ex{link, g.blocks, own, all, &bad};
     if (bad)
     {
         if (blockIdx.x == 0 && tid == 0) st->done = KRYLOV_ABORTED;
@@ -924,7 +926,7 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_small_kernel(ROWS rows, 
         reinterpret_cast<int32_t*>(part + (!ROWS::kSliced ? kCsrChunk : g.wps > 1 ? g.rows * g.wps : 0));
     rows.begin(g, first_row);
     __syncthreads();
-    grid_exchange ex{link, g.blocks, own, all, &bad};
+    grid_exchange<> ex{link, g.blocks, own, all, &bad};
     if (bad)
     {
         if (blockIdx.x == 0 && tid == 0) st->done = KRYLOV_ABORTED;
@@ -1065,7 +1067,7 @@ __global__ __launch_bounds__(kGridThreads) void bicg_grid_kernel(ROWS rows, grid
         reinterpret_cast<int32_t*>(part + (!ROWS::kSliced ? kCsrChunk : g.wps > 1 ? g.rows * g.wps : 0));
     rows.begin(g, first_row);
     __syncthreads();
-    grid_exchange ex{link, g.blocks, own, all, &bad};
+    grid_exchange<> ex{link, g.blocks, own, all, &bad};
     if (bad)
     {
         if (blockIdx.x == 0 && tid == 0) st->done = KRYLOV_ABORTED;
@@ -1207,4 +1209,154 @@ __global__ __launch_bounds__(kGridThreads) void bicg_grid_kernel(ROWS rows, grid
         *st = s;
     }
 }
+
+// ------------------------------------------------------- the vector part of an iteration
+// The scalars and vectors of one iteration between two products of the launch loops, in one launch
+// in place of three (totals, r update, x and p update): the total of p.Ap from the product's partials,
+// r -= alpha A p with r.z (and r.r), the exchange of those sums, and x += alpha p, p = z + beta p.  r
+// stays in registers between the two halves, x and p are requested ahead of the exchange: 7 vector
+// passes instead of 8 (FP32 on the Jacobi-scaled copy, z = r), 8 instead of 10 (FP64).  Two
+// workgroups' worth of a compute unit's registers; a thread's elements past its kVectorKeep groups are
+// read again.  DECIDE: the scalar rules of the loop, s <- the next state, returns beta.
+constexpr int kVectorThreads = 1024;
+constexpr int kVectorKeep = 3; // 16-byte groups of each vector that a thread keeps
+
+template <typename T, bool PRECOND, bool RR, typename DECIDE>
+__device__ __forceinline__ void vector_iteration(int64_t n, T* __restrict__ r, const T* __restrict__ Ap,
+                                                 const T* __restrict__ minv, T* __restrict__ x, T* __restrict__ p,
+                                                 const double* __restrict__ part_pAp, int npart,
+                                                 const krylov_state* __restrict__ st, krylov_state* __restrict__ st_next,
+                                                 grid_link link, DECIDE decide)
+{
+    constexpr int W = 16 / int(sizeof(T)), WAVES = kVectorThreads / 64;
+    typedef T vec_t __attribute__((ext_vector_type(W)));
+    __shared__ double own[2][2][WAVES], all[2][2][WAVES];
+    __shared__ int bad;
+    int const tid = threadIdx.x;
+    krylov_state s = *st;
+    if (s.done)
+    {
+        if (blockIdx.x == 0 && tid == 0) *st_next = s;
+        return;
+    }
+    if (tid == 0) bad = __hip_atomic_load(&link.mark->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    double const alpha_d = s.rz / reduce_partials<kVectorThreads>(part_pAp, npart); // a barrier for `bad` too
+    T const alpha = T(alpha_d);
+    if (bad)
+    {
+        if (blockIdx.x == 0 && tid == 0)
+        {
+            s.done = KRYLOV_ABORTED;
+            *st_next = s;
+        }
+        return;
+    }
+    grid_exchange<WAVES> ex{link, int(gridDim.x), own, all, &bad};
+    int64_t beg, end;
+    xcd_chunk_aligned<W>(n, beg, end);
+    int64_t const full = beg + (end - beg) / W * W;
+    double v[2] = {0.0, 0.0};
+    // element of r -> its new value, its products into the sums
+    auto half1 = [&](T ri, T api, T mi) {
+        ri = ri - alpha * api;
+        if constexpr (PRECOND)
+        {
+            T const zi = mi * ri;
+            v[0] += double(ri) * double(zi);
+            if constexpr (RR) v[1] += double(ri) * double(ri);
+        }
+        else
+            v[0] += double(ri) * double(ri);
+        return ri;
+    };
+    vec_t rk[kVectorKeep], xk[kVectorKeep], pk[kVectorKeep], mk[kVectorKeep];
+#pragma unroll
+    for (int g = 0; g < kVectorKeep; ++g)
+    {
+        int64_t const i = beg + (int64_t(g) * kVectorThreads + tid) * W;
+        if (i >= full) break;
+        rk[g] = *reinterpret_cast<const vec_t*>(r + i);
+        vec_t const av = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(Ap + i));
+        if constexpr (PRECOND) mk[g] = *reinterpret_cast<const vec_t*>(minv + i);
+        xk[g] = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(x + i));
+        pk[g] = *reinterpret_cast<const vec_t*>(p + i);
+#pragma unroll
+        for (int k = 0; k < W; ++k) rk[g][k] = half1(rk[g][k], av[k], PRECOND ? mk[g][k] : T(1));
+    }
+    for (int64_t i = beg + (int64_t(kVectorKeep) * kVectorThreads + tid) * W; i < full; i += kVectorThreads * W)
+    {
+        vec_t rv = *reinterpret_cast<const vec_t*>(r + i);
+        vec_t const av = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(Ap + i));
+        vec_t mv{};
+        if constexpr (PRECOND) mv = *reinterpret_cast<const vec_t*>(minv + i);
+#pragma unroll
+        for (int k = 0; k < W; ++k) rv[k] = half1(rv[k], av[k], PRECOND ? mv[k] : T(1));
+        *reinterpret_cast<vec_t*>(r + i) = rv;
+    }
+    // the last entries of the system, fewer than W
+    for (int64_t i = full + tid; i < end; i += kVectorThreads) r[i] = half1(r[i], Ap[i], PRECOND ? minv[i] : T(1));
+    if (!ex.template sum<RR ? 2 : 1>(v))
+    {
+        if (blockIdx.x == 0 && tid == 0)
+        {
+            s.done = KRYLOV_ABORTED;
+            *st_next = s;
+        }
+        return;
+    }
+    T const beta = T(decide(s, v[1], v[0]));
+    bool const more = s.done == KRYLOV_RUNNING;
+#pragma unroll
+    for (int g = 0; g < kVectorKeep; ++g)
+    {
+        int64_t const i = beg + (int64_t(g) * kVectorThreads + tid) * W;
+        if (i >= full) break;
+        *reinterpret_cast<vec_t*>(r + i) = rk[g];
+        vec_t xv = xk[g], pv = pk[g];
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+        {
+            xv[k] = xv[k] + alpha * pv[k];
+            pv[k] = (PRECOND ? mk[g][k] * rk[g][k] : rk[g][k]) + beta * pv[k];
+        }
+        __builtin_nontemporal_store(xv, reinterpret_cast<vec_t*>(x + i));
+        if (more) *reinterpret_cast<vec_t*>(p + i) = pv;
+    }
+    for (int64_t i = beg + (int64_t(kVectorKeep) * kVectorThreads + tid) * W; i < full; i += kVectorThreads * W)
+    {
+        vec_t const rv = *reinterpret_cast<const vec_t*>(r + i);
+        vec_t xv = __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(x + i));
+        vec_t pv = *reinterpret_cast<const vec_t*>(p + i), mv{};
+        if constexpr (PRECOND) mv = *reinterpret_cast<const vec_t*>(minv + i);
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+        {
+            xv[k] = xv[k] + alpha * pv[k];
+            pv[k] = (PRECOND ? mv[k] * rv[k] : rv[k]) + beta * pv[k];
+        }
+        __builtin_nontemporal_store(xv, reinterpret_cast<vec_t*>(x + i));
+        if (more) *reinterpret_cast<vec_t*>(p + i) = pv;
+    }
+    for (int64_t i = full + tid; i < end; i += kVectorThreads)
+    {
+        T const pi = p[i];
+        x[i] = x[i] + alpha * pi;
+        if (more) p[i] = (PRECOND ? minv[i] * r[i] : r[i]) + beta * pi;
+    }
+    if (blockIdx.x == 0 && tid == 0) *st_next = s;
+}
+
+// FP64 CG (cg_update_xr_kernel and cg_update_p_kernel)
+__global__ __launch_bounds__(kVectorThreads) void cg_vector_kernel(int64_t n, double* r, const double* Ap,
+                                                                   const double* minv, double* x, double* p,
+                                                                   const double* part_pAp, int npart,
+                                                                   const krylov_state* st, krylov_state* st_next,
+                                                                   grid_link link, int criterion, double tol,
+                                                                   int max_it);
+// mixed CG on the Jacobi-scaled copy, an iteration without a reliable update
+// (mixed_update_xr_kernel<true, false> and mixed_update_p_kernel<true> with decided = 0)
+__global__ __launch_bounds__(kVectorThreads) void mixed_vector_kernel(int64_t n, float* r, const float* Ap, float* x,
+                                                                      float* p, const double* part_pAp, int npart,
+                                                                      const krylov_state* st, krylov_state* st_next,
+                                                                      grid_link link, int max_it);
 } // namespace neon_amd

@@ -5,10 +5,42 @@
 
 #include <algorithm>
 #include <condition_variable>
+#include <memory>
 #include <mutex>
 
 namespace neon_amd
 {
+__global__ __launch_bounds__(kVectorThreads) void cg_vector_kernel(int64_t n, double* r, const double* Ap,
+                                                                   const double* minv, double* x, double* p,
+                                                                   const double* part_pAp, int npart,
+                                                                   const krylov_state* st, krylov_state* st_next,
+                                                                   grid_link link, int criterion, double tol,
+                                                                   int max_it)
+{
+    vector_iteration<double, true, true>(n, r, Ap, minv, x, p, part_pAp, npart, st, st_next, link,
+                                         [&](krylov_state& s, double rr, double rz) {
+                                             return cg_decide(s, rr, rz, criterion, tol, max_it);
+                                         });
+}
+
+__global__ __launch_bounds__(kVectorThreads) void mixed_vector_kernel(int64_t n, float* r, const float* Ap, float* x,
+                                                                      float* p, const double* part_pAp, int npart,
+                                                                      const krylov_state* st, krylov_state* st_next,
+                                                                      grid_link link, int max_it)
+{
+    vector_iteration<float, false, false>(n, r, Ap, nullptr, x, p, part_pAp, npart, st, st_next, link,
+                                          [&](krylov_state& s, double, double rz) {
+                                              double const beta = rz / s.rz;
+                                              int32_t const it = s.it + 1;
+                                              s.done = it >= max_it ? KRYLOV_LIMIT : KRYLOV_RUNNING;
+                                              if (!isfinite(rz)) s.done = KRYLOV_NONFINITE;
+                                              s.rz = rz;
+                                              s.it = it;
+                                              s.refine = 0;
+                                              return beta;
+                                          });
+}
+
 namespace
 {
 constexpr int64_t kGridLds = 160 * 1024 - 1024; // LDS of a compute unit less the static arrays
@@ -46,6 +78,9 @@ private:
     int used_ = 0;
 };
 
+
+} // namespace
+
 class unit_hold
 {
 public:
@@ -59,6 +94,13 @@ private:
     int count_;
 };
 
+std::shared_ptr<unit_hold> hold_units(int device, int count, int units)
+{
+    return std::make_shared<unit_hold>(device, count, units);
+}
+
+namespace
+{
 // The vectors of a loop's recurrence: all of them in LDS, or the fewest that must be (0: all), and the
 // most rows per thread in either case
 struct vector_need
@@ -216,6 +258,40 @@ bool krylov_engine::grid_run(Batch&& batch)
     return false;
 }
 
+int krylov_engine::vector_blocks(int64_t n, int width)
+{
+    grid_begin();
+    if (!grid_units_) return 0;
+    // at least one 16-byte group per thread, a multiple of 8 (the XCDs' shares) from 8 on
+    int64_t const b = std::min<int64_t>((n + int64_t(kVectorThreads) * width - 1) / (int64_t(kVectorThreads) * width),
+                                        std::min(grid_units_, kGridMaxBlocks));
+    return int(b >= 8 ? b / 8 * 8 : b);
+}
+
+void krylov_engine::cg_vector(int blocks, int64_t n, double* r, const double* Ap, const double* minv, double* x,
+                              double* p, const double* part, int npart, const krylov_state* st, krylov_state* next,
+                              int criterion, double tol, int32_t max_it)
+{
+    cg_vector_kernel<<<blocks, kVectorThreads, 0, s_>>>(n, r, Ap, minv, x, p, part, npart, st, next, grid_next(1),
+                                                        criterion, tol, max_it);
+}
+
+void krylov_engine::mixed_vector(int blocks, int64_t n, float* r, const float* Ap, float* x, float* p,
+                                 const double* part, int npart, const krylov_state* st, krylov_state* next,
+                                 int32_t max_it)
+{
+    mixed_vector_kernel<<<blocks, kVectorThreads, 0, s_>>>(n, r, Ap, x, p, part, npart, st, next, grid_next(1), max_it);
+}
+
+bool krylov_engine::vector_gave_up()
+{
+    NEON_CHECK_HIP(hipMemcpyAsync(host_ring_, state_.data() + 3, sizeof(krylov_state), hipMemcpyDeviceToHost, s_));
+    NEON_CHECK_HIP(hipStreamSynchronize(s_));
+    if (!host_ring_[0].done) return false;
+    grid_clear();
+    return true;
+}
+
 bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion,
                               double tol, int32_t max_it, const krylov_work* work, solve_result& out)
 {
@@ -248,7 +324,7 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
     int const iters = int(std::min<int64_t>(few ? buffers / 2 : buffers, 64));
     if (iters < 1) return false;
     krylov_state* st = state_.data() + 2;
-    unit_hold const hold(grid_device_, g.blocks, grid_units_);
+    auto const hold = hold_units(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto kernel, auto rows) {
         allow_lds(kernel, g.lds);
         return grid_run([&, kernel](bool first) {
@@ -328,7 +404,7 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
     if (iters < 1) return false;
     int const cuda_rule = criterion == NEON_STOP_ABSOLUTE_PRECONDITIONED ? 1 : 0;
     krylov_state* st = state_.data() + 2;
-    unit_hold const hold(grid_device_, g.blocks, grid_units_);
+    auto const hold = hold_units(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto rows) {
         auto kernel = bicg_grid_kernel<decltype(rows)>;
         allow_lds(kernel, g.lds);

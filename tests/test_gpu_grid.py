@@ -163,8 +163,9 @@ def test_cg_ends(ctx, criterion):
 
 
 def test_a_grid_that_gives_up_is_solved_by_launches(ctx):
-    """With no patience the first wait of a workgroup for another ends the grid; the solve then
-    takes the launch-per-phase loop, and the next one with patience the grid again."""
+    """With no patience the first wait of a workgroup for another ends the grid, and then the one-launch
+    vector part of the launch loop; the solve takes separate launches, and the next one with
+    patience the grid again.  The same for the mixed loop."""
     fn = _capi.measure_lib().neon_test_grid_patience
     fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.c_int64]
     A, b = _spd(40000, 20, 8)
@@ -172,15 +173,43 @@ def test_a_grid_that_gives_up_is_solved_by_launches(ctx):
     def solve():
         return _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b)
 
+    mg, bm = _mesh(ctx, (30, 29, 31), "grid", 0.0)
+    mg.assemble(neon_amd.PRECISION_MIXED)
+    mg.enforce_dirichlet(problems.block_rollers(31, dims=(30, 29, 31)).fixed_dofs(), bm)
+
+    def mixed():
+        return mg.solve(bm, tol=1e-10)
+
     grid, launches = _both(ctx, solve)
+    patient = mixed()
     ctx.check(fn(ctx.handle, 0))
     try:
-        impatient = solve()
+        impatient, impatient_mixed = solve(), mixed()
     finally:
         ctx.check(fn(ctx.handle, 10 ** 8))
-    assert np.array_equal(impatient[0], launches[0]) and impatient[1] == launches[1]
+    _check(A, b, impatient, launches)
+    _check(_matrix(mg), bm, impatient_mixed, patient)
     again = solve()
     assert np.array_equal(again[0], grid[0]) and again[1] == grid[1]
+    assert np.array_equal(mixed()[0], patient[0])
+
+
+# one workgroup, its last entries fewer than a 16-byte group; several; and more entries than the
+# threads keep in registers
+@pytest.mark.parametrize("dims", [(1, 1, 1), (7, 6, 5), (20, 19, 23), (44, 43, 45), (104, 102, 101)])
+def test_mixed_cg_vector_part(ctx, dims):
+    """The mixed loop's one-launch vector part: the true residual against the FP32 tangent, and the
+    FP64 solve's iteration count (reliable updates keep the Krylov space: within 25 % and 8, the
+    test's period)."""
+    print(dims, flush=True)
+    mg, b = _mesh(ctx, dims, "grid", 0.0)
+    its64 = mg.solve(b, tol=1e-8)[1]
+    p = problems.block_rollers(max(dims), dims=dims)
+    mg.assemble(neon_amd.PRECISION_MIXED)
+    mg.enforce_dirichlet(p.fixed_dofs(), b)
+    x, its, _ = mg.solve(b, tol=1e-8)
+    assert np.linalg.norm(b - _matrix(mg) @ x) <= 1.1e-8 * np.linalg.norm(b)
+    assert its <= 1.25 * its64 + 8, (its, its64)
 
 
 def test_two_contexts_share_the_gpu():
