@@ -1061,21 +1061,25 @@ __global__ __launch_bounds__(64) void assemble_mass_kernel(const int32_t* __rest
 // ----------------------------------------------------------------- Dirichlet
 // For each fixed dof d: zero row d and column d except the diagonal.  All writes are
 // zeros and the diagonal is never written, so concurrent dofs need no ordering; the
-// result equals the sequential loop of enforce_dirichlet_conditions.
+// result equals the sequential loop of enforce_dirichlet_conditions.  One wavefront per dof, a lane
+// per block of the dof's node, which finds the node among its column node's blocks by bisection (one
+// thread per dof, scanning both rows, waited for some 700 loads in turn: 57 us per call at 363 and
+// at 3,072 dofs alike, 3.8 us here).
 template <typename KT>
 __global__ __launch_bounds__(kBlock) void dirichlet_kernel(int32_t n_fixed, const int32_t* __restrict__ fixed,
                                                            const int32_t* __restrict__ bptr,
                                                            const int32_t* __restrict__ bcol, KT* __restrict__ K,
                                                            double* __restrict__ b)
 {
-    int32_t const t = blockIdx.x * kBlock + threadIdx.x;
+    int32_t const t = int32_t((int64_t(blockIdx.x) * kBlock + threadIdx.x) >> 6);
+    int const lane = threadIdx.x & 63;
     if (t >= n_fixed) return;
     int32_t const d = fixed[t];
     int32_t const nd = d / 3, i = d % 3;
     int32_t const b0 = bptr[nd];
     int32_t const deg = bptr[nd + 1] - b0;
-    if (b) b[d] = 0.0;
-    for (int32_t s = 0; s < deg; ++s)
+    if (b && lane == 0) b[d] = 0.0;
+    for (int32_t s = lane; s < deg; s += 64)
     {
         int32_t const m = bcol[b0 + s];
         // row d: entries (i, j) of block (nd, m)
@@ -1084,22 +1088,25 @@ __global__ __launch_bounds__(kBlock) void dirichlet_kernel(int32_t n_fixed, cons
             if (m == nd && j == i) continue;
             K[9ll * b0 + 3ll * i * deg + 3ll * s + j] = KT(0);
         }
-        // column d in the rows of node m: find the slot of nd in m's block row
+        // column d in the rows of node m: the slot of nd in m's block row (ascending columns; the
+        // pattern is symmetric, so it is there)
         int32_t const c0 = bptr[m];
         int32_t const cdeg = bptr[m + 1] - c0;
-        int32_t slot = -1;
-        for (int32_t q = 0; q < cdeg; ++q)
-            if (bcol[c0 + q] == nd)
-            {
-                slot = q;
-                break;
-            }
-        if (slot < 0) continue;
+        int32_t lo = 0, hi = cdeg - 1;
+        while (lo < hi)
+        {
+            int32_t const mid = (lo + hi) >> 1;
+            if (bcol[c0 + mid] < nd)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        if (bcol[c0 + lo] != nd) continue;
         // column d: entries (j, i) of block (m, nd)
         for (int j = 0; j < 3; ++j)
         {
             if (m == nd && j == i) continue;
-            K[9ll * c0 + 3ll * j * cdeg + 3ll * slot + i] = KT(0);
+            K[9ll * c0 + 3ll * j * cdeg + 3ll * lo + i] = KT(0);
         }
     }
 }

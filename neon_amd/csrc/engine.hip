@@ -242,6 +242,7 @@ krylov_engine::krylov_engine(hipStream_t s) : s_(s)
     // two ping-ponged states; the resident grids' state and their abort word
     state_.resize(4);
     scalar_.resize(1);
+    norms_.resize(4);
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_state_), sizeof(krylov_state)));
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ring_), 4 * sizeof(krylov_state)));
     for (auto& e : ring_events_) NEON_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -290,6 +291,19 @@ double krylov_engine::dot(int64_t n, const double* a, const double* b)
     NEON_CHECK_HIP(hipMemcpyAsync(host_scalar_, scalar_.data(), sizeof(double), hipMemcpyDeviceToHost, s_));
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
     return *host_scalar_;
+}
+
+void krylov_engine::step_norms(int64_t n, double* u, const double* d, const double* f, const double* r, double* out)
+{
+    int const nb = vec_blocks(n);
+    step_norms_kernel<<<nb, kBlock, 0, s_>>>(n, u, d, f, r, part_[0].data(), part_[1].data(), part_[2].data(),
+                                             part_[3].data());
+    step_norms_reduce_kernel<<<4, kBlock, 0, s_>>>(part_[0].data(), part_[1].data(), part_[2].data(), part_[3].data(),
+                                                   nb, norms_.data());
+    NEON_CHECK_HIP(hipGetLastError());
+    NEON_CHECK_HIP(hipMemcpyAsync(host_state_, norms_.data(), 4 * sizeof(double), hipMemcpyDeviceToHost, s_));
+    NEON_CHECK_HIP(hipStreamSynchronize(s_));
+    std::memcpy(out, host_state_, 4 * sizeof(double));
 }
 
 void krylov_engine::jacobi64(const linear_operator& A, double* minv, int eigen_rule)
@@ -1354,7 +1368,7 @@ void device_mesh::enforce_dirichlet_mass(int32_t n_fixed, const int32_t* fixed_d
 {
     if (n_fixed <= 0) return;
     if (!m64_valid_) throw status_error(NEON_BAD_ARGUMENT, "no mass matrix assembled");
-    dirichlet_kernel<double><<<grid_for(n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
+    dirichlet_kernel<double><<<grid_for(64ll * n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
                                                                      m64_.data(), nullptr);
     NEON_CHECK_HIP(hipGetLastError());
 }
@@ -1385,10 +1399,10 @@ void device_mesh::enforce_dirichlet(int32_t n_fixed, const int32_t* fixed_dev, d
     if (n_fixed <= 0) return;
     s64_fresh_ = s32_fresh_ = y64_fresh_ = y32_fresh_ = y32s_fresh_ = false;
     if (precision == NEON_PRECISION_FP64)
-        dirichlet_kernel<double><<<grid_for(n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
+        dirichlet_kernel<double><<<grid_for(64ll * n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
                                                                          k64_.data(), b_dev);
     else
-        dirichlet_kernel<float><<<grid_for(n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
+        dirichlet_kernel<float><<<grid_for(64ll * n_fixed), kBlock, 0, s_>>>(n_fixed, fixed_dev, bptr_.data(), bcol_.data(),
                                                                         k32_.data(), b_dev);
     NEON_CHECK_HIP(hipGetLastError());
 }

@@ -232,6 +232,8 @@ public:
     bool all_positive(int64_t n, const double* v);
 
     double dot(int64_t n, const double* a, const double* b);
+    // u += d, then out = u.u, d.d, f.f, r.r (synchronises)
+    void step_norms(int64_t n, double* u, const double* d, const double* f, const double* r, double* out);
 
     hipStream_t stream() const { return s_; }
     int vec_blocks(int64_t n) const;
@@ -296,7 +298,7 @@ private:
     device_array<uint64_t> grid_slots_;
     device_array<double> grid_ring_, grid_r_, grid_bicg_;
     double* host_scalar_ = nullptr;
-    device_array<double> scalar_;
+    device_array<double> scalar_, norms_;
     int64_t n_ = 0, n_mixed_ = 0;
     device_array<double> r_, p_, Ap_;
     device_array<double> r0_, v_, s_vec_, t_, ph_, sh_;

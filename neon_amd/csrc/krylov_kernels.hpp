@@ -995,6 +995,51 @@ __global__ __launch_bounds__(kBlock) void dot_kernel(int64_t n, const double* __
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
+// A Newton iteration's displacement step u += d with the partials of its four norms (u.u, d.d, f.f,
+// r.r), and their totals: two launches and one wait in place of nine and four.
+__global__ __launch_bounds__(kBlock) void step_norms_kernel(int64_t n, double* __restrict__ u,
+                                                            const double* __restrict__ d,
+                                                            const double* __restrict__ f,
+                                                            const double* __restrict__ r, double* __restrict__ part_u,
+                                                            double* __restrict__ part_d, double* __restrict__ part_f,
+                                                            double* __restrict__ part_r)
+{
+    int64_t beg, end;
+    xcd_chunk(n, beg, end);
+    double su = 0.0, sd = 0.0, sf = 0.0, sr = 0.0;
+    for (int64_t i = beg + threadIdx.x; i < end; i += kBlock)
+    {
+        double const di = d[i], ui = u[i] + di, fi = f[i], ri = r[i];
+        u[i] = ui;
+        su += ui * ui;
+        sd += di * di;
+        sf += fi * fi;
+        sr += ri * ri;
+    }
+    su = block_sum<kBlock>(su);
+    sd = block_sum<kBlock>(sd);
+    sf = block_sum<kBlock>(sf);
+    sr = block_sum<kBlock>(sr);
+    if (threadIdx.x == 0)
+    {
+        part_u[blockIdx.x] = su;
+        part_d[blockIdx.x] = sd;
+        part_f[blockIdx.x] = sf;
+        part_r[blockIdx.x] = sr;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void step_norms_reduce_kernel(const double* __restrict__ part_u,
+                                                                   const double* __restrict__ part_d,
+                                                                   const double* __restrict__ part_f,
+                                                                   const double* __restrict__ part_r, int npart,
+                                                                   double* __restrict__ out)
+{
+    const double* const part[4] = {part_u, part_d, part_f, part_r};
+    double const s = reduce_partials<kBlock>(part[blockIdx.x], npart);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
 __global__ __launch_bounds__(kBlock) void reduce_to_kernel(const double* __restrict__ part, int npart,
                                                            double* __restrict__ out)
 {

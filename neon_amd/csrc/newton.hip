@@ -357,8 +357,10 @@ int newton_solve(neon_context* ctx, const neon_newton_options* o, int32_t n_bc, 
                     break;
                 }
                 t0 = std::chrono::steady_clock::now();
-                add_kernel<<<blocks(n), kBlock, 0, s>>>(n, delta.data(), u);
-                NEON_CHECK_HIP(hipGetLastError());
+                // the step and the norms of update_relative_norms (static_matrix.hpp:385-400); f_int
+                // and the residual are those of the iteration's start
+                double sq[4];
+                k.step_norms(n, u, delta.data(), m.f_int(), mres.data(), sq);
                 err = m.update_internal_variables(u);
                 tm.update_ms += ms_since(t0);
                 if (err != NEON_OK)
@@ -366,11 +368,7 @@ int newton_solve(neon_context* ctx, const neon_newton_options* o, int32_t n_bc, 
                     record(it, sr.iterations, err, 0, 0);
                     break;
                 }
-                // update_relative_norms (static_matrix.hpp:385-400)
-                double const un = std::sqrt(k.dot(n, u, u));
-                double const fi = std::sqrt(k.dot(n, m.f_int(), m.f_int()));
-                double const dn = std::sqrt(k.dot(n, delta.data(), delta.data()));
-                double const rn = std::sqrt(k.dot(n, mres.data(), mres.data()));
+                double const un = std::sqrt(sq[0]), dn = std::sqrt(sq[1]), fi = std::sqrt(sq[2]), rn = std::sqrt(sq[3]);
                 bool const rel = o->norm_mode == 1 ? true
                                                    : (!o->absolute_norm && !is_approx(un, 0.0, 1.0)
                                                       && !is_approx(std::max(fe, fi), 0.0, 1.0));
