@@ -969,6 +969,17 @@ device_mesh::device_mesh(hipStream_t s, int32_t n_nodes, const double* X, int32_
         for (int64_t e = 0; e < E_; ++e) elems[fill[colour[e]]++] = int32_t(e);
     }
 
+    // the incidence with each element's local node, 8 e + a (staged assembly)
+    if (int64_t(E_) <= kStageElements)
+    {
+        std::vector<int32_t> fill(inc_ptr.begin(), inc_ptr.end() - 1);
+        for (int64_t e = 0; e < E_; ++e)
+            for (int a = 0; a < 8; ++a) inc[fill[conn[8 * e + a]]++] = int32_t(8 * e + a);
+        incp_.resize(inc_ptr.size());
+        inc_.resize(inc.size());
+        NEON_CHECK_HIP(hipMemcpyAsync(incp_.data(), inc_ptr.data(), inc_ptr.size() * sizeof(int32_t), hipMemcpyHostToDevice, s_));
+        NEON_CHECK_HIP(hipMemcpyAsync(inc_.data(), inc.data(), inc.size() * sizeof(int32_t), hipMemcpyHostToDevice, s_));
+    }
     X_.resize(3ull * N_);
     u_.resize(3ull * N_);
     fint_.resize(3ull * N_);
@@ -1260,32 +1271,59 @@ void device_mesh::save_internal_variables(bool converged)
     NEON_CHECK_HIP(hipGetLastError());
 }
 
-void device_mesh::assemble(const double* u_dev, int precision)
+// Every element's blocks and forces at once, then their sums by node
+void device_mesh::assemble_staged(const double* u_dev, qp_state const& st, bool fp64)
 {
-    int64_t const Q = 8ll * E_;
-    qp_state st{sigma_.data(), coef_.data(), detF_.data(), eps_p_.data(), ebar_.data(), vm_.data(), Q,
-                eps_p_old_.data(), ebar_old_.data(), age_.data(), age_old_.data()};
-    bool const finite = is_finite_model(model_); // is_finite_deformation()
+    bool const finite = is_finite_model(model_);
     bool const general = model_ == NEON_MODEL_J2_DAMAGE;
     bool const full = is_microsphere(model_);
-    // neon integrates the small-strain models on the current configuration (submesh.cpp:68,84);
-    // the consistent mode integrates them on X
-    if (!finite && tangent_mode_ == NEON_TANGENT_CONSISTENT) u_dev = nullptr;
-    hipEvent_t e0, e1;
-    NEON_CHECK_HIP(hipEventCreate(&e0));
-    NEON_CHECK_HIP(hipEventCreate(&e1));
-    NEON_CHECK_HIP(hipEventRecord(e0, s_));
-    NEON_CHECK_HIP(hipMemsetAsync(fint_.data(), 0, 3ull * N_ * sizeof(double), s_));
-    if (precision == NEON_PRECISION_FP64)
+    stage_.resize(size_t(E_) * (576 + 24));
+    double* const kb = stage_.data();
+    double* const fb = kb + size_t(E_) * 576;
+    int dev = 0, cus = 256;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    int const blocks = int(std::min<int64_t>(E_, int64_t(cus) * assembly_blocks_per_cu));
+#define NEON_STAGE(FIN, FULL, GEN)                                                                                 \
+    assemble_kernel<double, FIN, FULL, GEN, true><<<blocks, 64, 0, s_>>>(nullptr, E_, conn_.data(), X_.data(), u_dev, \
+                                                                         st, nullptr, nullptr, nullptr, nullptr, kb, fb)
+    if (general)
+        NEON_STAGE(false, true, true);
+    else if (full)
+        NEON_STAGE(true, true, false);
+    else if (finite)
+        NEON_STAGE(true, false, false);
+    else
+        NEON_STAGE(false, false, false);
+#undef NEON_STAGE
+    NEON_CHECK_HIP(hipGetLastError());
+    // the values past nnz stay zero (kValuePad)
+    if (fp64)
     {
-        k64_.resize(nnz_ + kValuePad);
-        NEON_CHECK_HIP(hipMemsetAsync(k64_.data(), 0, (nnz_ + kValuePad) * sizeof(double), s_));
+        fill_zero(s_, kValuePad, k64_.data() + nnz_);
+        assemble_gather_kernel<double><<<grid_for(32ll * N_), kBlock, 0, s_>>>(
+            N_, incp_.data(), inc_.data(), slots_.data(), bptr_.data(), kb, fb, k64_.data(), fint_.data());
     }
     else
     {
-        k32_.resize(nnz_ + kValuePad);
-        NEON_CHECK_HIP(hipMemsetAsync(k32_.data(), 0, (nnz_ + kValuePad) * sizeof(float), s_));
+        NEON_CHECK_HIP(hipMemsetAsync(k32_.data() + nnz_, 0, kValuePad * sizeof(float), s_));
+        assemble_gather_kernel<float><<<grid_for(32ll * N_), kBlock, 0, s_>>>(
+            N_, incp_.data(), inc_.data(), slots_.data(), bptr_.data(), kb, fb, k32_.data(), fint_.data());
     }
+    NEON_CHECK_HIP(hipGetLastError());
+}
+
+// One colour of elements after the other, into the cleared tangent
+void device_mesh::assemble_coloured(const double* u_dev, qp_state const& st, bool fp64)
+{
+    bool const finite = is_finite_model(model_); // is_finite_deformation()
+    bool const general = model_ == NEON_MODEL_J2_DAMAGE;
+    bool const full = is_microsphere(model_);
+    NEON_CHECK_HIP(hipMemsetAsync(fint_.data(), 0, 3ull * N_ * sizeof(double), s_));
+    if (fp64)
+        NEON_CHECK_HIP(hipMemsetAsync(k64_.data(), 0, (nnz_ + kValuePad) * sizeof(double), s_));
+    else
+        NEON_CHECK_HIP(hipMemsetAsync(k32_.data(), 0, (nnz_ + kValuePad) * sizeof(float), s_));
     int dev = 0, cus = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1301,14 +1339,14 @@ void device_mesh::assemble(const double* u_dev, int precision)
                                                           bptr_.data(), K, fint_.data())
         if (general)
         {
-            if (precision == NEON_PRECISION_FP64)
+            if (fp64)
                 assemble_kernel<double, false, true, true><<<blocks, 64, 0, s_>>>(
                     el, cnt, conn_.data(), X_.data(), u_dev, st, slots_.data(), bptr_.data(), k64_.data(), fint_.data());
             else
                 assemble_kernel<float, false, true, true><<<blocks, 64, 0, s_>>>(
                     el, cnt, conn_.data(), X_.data(), u_dev, st, slots_.data(), bptr_.data(), k32_.data(), fint_.data());
         }
-        else if (precision == NEON_PRECISION_FP64)
+        else if (fp64)
         {
             if (full)
                 NEON_ASSEMBLE(double, true, true, k64_.data());
@@ -1328,6 +1366,32 @@ void device_mesh::assemble(const double* u_dev, int precision)
         }
 #undef NEON_ASSEMBLE
     }
+    NEON_CHECK_HIP(hipGetLastError());
+}
+
+void device_mesh::assemble(const double* u_dev, int precision)
+{
+    int64_t const Q = 8ll * E_;
+    qp_state st{sigma_.data(), coef_.data(), detF_.data(), eps_p_.data(), ebar_.data(), vm_.data(), Q,
+                eps_p_old_.data(), ebar_old_.data(), age_.data(), age_old_.data()};
+    bool const finite = is_finite_model(model_); // is_finite_deformation()
+    // neon integrates the small-strain models on the current configuration (submesh.cpp:68,84);
+    // the consistent mode integrates them on X
+    if (!finite && tangent_mode_ == NEON_TANGENT_CONSISTENT) u_dev = nullptr;
+    hipEvent_t e0, e1;
+    NEON_CHECK_HIP(hipEventCreate(&e0));
+    NEON_CHECK_HIP(hipEventCreate(&e1));
+    NEON_CHECK_HIP(hipEventRecord(e0, s_));
+    bool const staged = int64_t(E_) <= kStageElements;
+    bool const fp64 = precision == NEON_PRECISION_FP64;
+    if (fp64)
+        k64_.resize(nnz_ + kValuePad);
+    else
+        k32_.resize(nnz_ + kValuePad);
+    if (staged)
+        assemble_staged(u_dev, st, fp64);
+    else
+        assemble_coloured(u_dev, st, fp64);
     NEON_CHECK_HIP(hipGetLastError());
     NEON_CHECK_HIP(hipEventRecord(e1, s_));
     NEON_CHECK_HIP(hipEventSynchronize(e1));

@@ -325,6 +325,13 @@ struct spmv_config
     int blocks32 = 0;
 };
 
+// Meshes of at most this many elements assemble through staged element blocks, 4,800 bytes each, which
+// then stay in the 256 MB cache between the two launches: 8^3, 16^3, 25^3, 32^3 elements 24, 43, 91,
+// 175 us (FP64) against 76, 90, 137, 233 us colour by colour.  Larger ones go colour by colour, which
+// moves less in FP32 and needs no scratch: 40^3 elements 365 us (FP32 298) against 382 (361) staged.
+constexpr int64_t kStageElements = int64_t(1) << 15;
+struct qp_state; // element_kernels.hpp
+
 // Device-resident mesh: geometry, constitutive state, pattern, tangent and f_int.
 class device_mesh
 {
@@ -437,6 +444,8 @@ public:
     kernel_profiler* prof = nullptr;
 
 private:
+    void assemble_staged(const double* u_dev, qp_state const& st, bool fp64);
+    void assemble_coloured(const double* u_dev, qp_state const& st, bool fp64);
     void build_sliced_pattern();
     void build_symmetric_pattern();
     sym_matrix sym_layout() const;
@@ -447,7 +456,8 @@ private:
     std::vector<int32_t> bptr_h_, bcol_h_;
     std::vector<int32_t> colour_offsets_;
     device_array<double> X_, u_, params_, fint_;
-    device_array<int32_t> conn_, elems_, bptr_, bcol_, self_slot_;
+    device_array<int32_t> conn_, elems_, bptr_, bcol_, self_slot_, incp_, inc_;
+    device_array<double> stage_; // staged assembly: element blocks, then element forces
     device_array<uint8_t> slots_;
     device_array<double> k64_, m64_;
     device_array<float> k32_;
