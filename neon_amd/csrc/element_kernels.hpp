@@ -802,7 +802,7 @@ __global__ __launch_bounds__(kBlock) void expand_tangent_kernel(int64_t Q, const
 // ------------------------------------------------------------------ assembly
 // One wavefront (= one 64-thread block) per element at a time; blocks stride over the
 // elements of one colour, so no two elements in flight share a node and the K / f_int
-// read-modify-writes need no atomics.
+// read-modify-writes need no atomics (or over all elements, staging their blocks: STAGE below).
 //
 // Per element:
 //   phase A, lane = (l, a): J_l = x dN_l (current configuration), det, inverse,

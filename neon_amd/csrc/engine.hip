@@ -361,14 +361,16 @@ void krylov_engine::run_batches(krylov_state* st, int64_t& launched, Batch&& bat
     NEON_CHECK_HIP(hipMemcpyAsync(host_state_, st + (launched & 1), sizeof(krylov_state), hipMemcpyDeviceToHost, s_));
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
 }
-// Jacobi-PCG in FP64.  Per iteration: SpMV fused with the block partials of p.Ap, their total
-// (one block: the SpMV has one partial per slice quadruple, which every update block would
-// otherwise reduce), the r update fused with the partials of r.r and r.z, and the x and p
-// updates with the convergence decision (each of its blocks reduces the r update's partials;
-// x += alpha p sits there because that kernel reads p anyway: 10 vector passes, not 11);
-// scalars stay on the device and the host polls the state every `poll_every` iterations (a
-// batch queued ahead of the one it waits on).
-// Iterations past convergence are no-ops, so the reported count is exact.
+
+// Jacobi-PCG in FP64: inside one resident grid where the system fits it (cg64_grid), otherwise by
+// launches.  Per iteration: SpMV fused with the block partials of p.Ap, then the vector part in one
+// launch (vector_iteration; 8 vector passes).  Where that is not available (kernel shapes, the
+// resident grid's units), three launches: the total of p.Ap (one block: the SpMV has one partial per
+// slice quadruple, which every update block would otherwise reduce), the r update fused with the
+// partials of r.r and r.z, and the x and p updates with the convergence decision (x += alpha p sits
+// there because that kernel reads p anyway: 10 vector passes, not 11).  Scalars stay on the device
+// and the host polls the state every `poll_every` iterations (a batch queued ahead of the one it
+// waits on).  Iterations past convergence are no-ops, so the reported count is exact.
 solve_result krylov_engine::cg64(const linear_operator& A, const double* b, double* x, const double* minv,
                                  int criterion, double tol, int32_t max_it, const krylov_work* work)
 {

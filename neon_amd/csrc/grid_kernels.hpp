@@ -1215,9 +1215,8 @@ __global__ __launch_bounds__(kGridThreads) void bicg_grid_kernel(ROWS rows, grid
 // in place of three (totals, r update, x and p update): the total of p.Ap from the product's partials,
 // r -= alpha A p with r.z (and r.r), the exchange of those sums, and x += alpha p, p = z + beta p.  r
 // stays in registers between the two halves, x and p are requested ahead of the exchange: 7 vector
-// passes instead of 8 (FP32 on the Jacobi-scaled copy, z = r), 8 instead of 10 (FP64).  Two
-// workgroups' worth of a compute unit's registers; a thread's elements past its kVectorKeep groups are
-// read again.  DECIDE: the scalar rules of the loop, s <- the next state, returns beta.
+// passes instead of 8 (FP32 on the Jacobi-scaled copy, z = r), 8 instead of 10 (FP64).  One workgroup
+// per compute unit; a thread's elements past its kVectorKeep groups are read again.  DECIDE: the scalar rules of the loop, s <- the next state, returns beta.
 constexpr int kVectorThreads = 1024;
 constexpr int kVectorKeep = 3; // 16-byte groups of each vector that a thread keeps
 
