@@ -9,7 +9,8 @@
 // matrix product plus two or three exchanges of 1.5 (32 workgroups) to 3 us (256 workgroups).
 // Per FP64 CG iteration on neo-Hooke blocks, launches against grid: 375 dofs 20.0 -> 6.1 us,
 // 27,783 24.6 -> 7.7, 59,049 26.7 -> 8.7, 117,912 31.9 -> 19.1, 311,469 48.6 -> 29.4, 680,943 72.9
-// -> 55.7, 1,167,051 114 -> 105.
+// -> 55.7; with the launches' vector part in one of them (vector_iteration) 50^3 cells 56.7 -> 43.7,
+// 64^3 88.3 -> 84.6.
 //
 // Visibility.  The only data that crosses workgroups are the exchanged scalars and the gathered
 // vector p.  Both are written with agent-scope (write-through) stores; a wavefront waits for its
