@@ -157,7 +157,9 @@ __global__ __launch_bounds__(kBlock) void spmv_nb_kernel(nb_matrix A, const VT* 
 // back: the slices in the opposite order.  A solver alternates it from product to product, so that a
 // product starts with the part of the matrix that the one before read last and the 256 MB
 // memory-side cache may still hold: 91^3 nodes, mixed precision 1,534 -> 1,397 ms per load step
-// (147 -> 134 us per iteration), 80^3 FP64 384 -> 355 ms per solve.
+// (147 -> 134 us per iteration), 80^3 FP64 384 -> 355 ms per solve.  Whole groups of 32 change places,
+// so that a slice stays on its XCD, whose L2 may hold it: 20^3, 28^3, 30^3 cells numbered by a mesh
+// generator, mixed, 90.5, 138.2, 154.2 ms with the XCD changing, 86.0, 133.1, 148.5 here.
 template <bool I16, bool NT, typename VT, typename XT, typename YT, typename AT, bool DOT, int MODE>
 __global__ __launch_bounds__(256) void spmv_sell_kernel(sell_matrix A, const VT* __restrict__ val,
                                                         const XT* __restrict__ x, YT* __restrict__ y,
@@ -170,7 +172,8 @@ __global__ __launch_bounds__(256) void spmv_sell_kernel(sell_matrix A, const VT*
     double dot = 0.0;
     for (int32_t q = int32_t(blockIdx.x) * 4 + wave; q < A.slices; q += int32_t(gridDim.x) * 4)
     {
-        int32_t const s = back ? A.slices - 1 - q : q;
+        int32_t const full = A.slices >> 5; // groups of 32 slices, four per workgroup on 8 XCDs
+        int32_t const s = back && q < full << 5 ? ((full - 1 - (q >> 5)) << 5) + (q & 31) : q;
         int32_t const node = A.snode[int64_t(s) * 64 + lane];
         bool const ok = node >= 0;
         int64_t const nn = ok ? int64_t(node) : -1 - int64_t(node);
