@@ -797,6 +797,8 @@ __global__ __launch_bounds__(kGridThreads) void cg_grid_kernel(ROWS rows, grid_s
         if (alive) s = cg_first_state(v[0], v[1], criterion, tol, max_it);
         if (s.done) iters = 0;
     }
+    else
+        __syncthreads(); // l_p whole before a lone workgroup gathers from it (the exchange is that barrier otherwise)
     for (int k = 0; alive && k < iters; ++k)
     {
         if (!ROWS::kSliced && g.blocks == 1) // local rows are the system's: p is gathered from LDS

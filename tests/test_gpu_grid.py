@@ -10,6 +10,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import scipy.sparse.linalg
 import scipy.sparse as sp
 
 import neon_amd
@@ -132,6 +133,66 @@ def test_cg_on_host_csr(ctx, n, per_row, long_rows):
     A, b = _spd(n, per_row, n, long_rows)
     grid, launches = _both(ctx, lambda: _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b))
     _check(A, b, grid, launches)
+
+
+def _chain(n, shift):
+    return sp.diags([-np.ones(n - 1), np.full(n, 2.0 + shift), -np.ones(n - 1)], [-1, 0, 1], format="csr")
+
+
+def _laplacian(m):
+    one = sp.identity(m)
+    return sp.csr_matrix(sp.kron(_chain(m, 0.0), one) + sp.kron(one, _chain(m, 0.0)))
+
+
+# Systems of one workgroup (at most 1,024 rows and 8,192 entries) whose solves take several launches
+# of 64 iterations: a continued launch gathers p from LDS, which it has filled from global memory.
+ONE_WORKGROUP = {"laplacian 30x30": lambda: _laplacian(30), "chain 1000": lambda: _chain(1000, 0.01),
+                 "chain 1024": lambda: _chain(1024, 0.01), "chain 65": lambda: _chain(65, 1e-4)}
+
+
+@pytest.mark.parametrize("name", ONE_WORKGROUP)
+def test_cg_of_one_workgroup_over_several_launches(ctx, name):
+    """The true residual differs from the recurrence's by at most eps |A| |x| per iteration (|A| <= 8);
+    each solve repeats bit for bit."""
+    print(name, flush=True)
+    A = ONE_WORKGROUP[name]()
+    b = np.random.default_rng(13).standard_normal(A.shape[0])
+    grid, launches = _both(ctx, lambda: _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b))
+    assert grid[1] > 64 or name == "chain 65"
+    for x, its, _ in (grid, launches):
+        drift = its * np.finfo(float).eps * 8.0 * np.linalg.norm(x)
+        assert np.linalg.norm(b - A @ x) <= 1e-10 * np.linalg.norm(b) + drift
+    assert abs(grid[1] - launches[1]) <= max(2, 0.02 * launches[1]), (grid[1], launches[1])
+    # other systems of one workgroup on the same compute units' LDS in between
+    for k in range(3):
+        other, c = _spd(700 + k, 5, 40 + k)
+        _solve_csr(ctx, neon_amd.conjugate_gradient_hip, other, c)
+        again = _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b)
+        assert np.array_equal(again[0], grid[0]) and again[1] == grid[1]
+
+
+@pytest.mark.parametrize("limit", [64, 65, 129])
+def test_cg_of_one_workgroup_stops_at_the_limit(ctx, limit):
+    """The limit at the end of a launch, and after the first iteration of the second and of the third
+    one.  The iterate that is left meets the a-priori bound of k conjugate gradient iterations,
+    |x_k - x|_A <= 2 ((sqrt(c) - 1) / (sqrt(c) + 1))^k |x|_A (the Jacobi scaling is by one number, and
+    c < 4.01 / 0.01 for this chain)."""
+    A = _chain(1000, 0.01)
+    b = np.random.default_rng(14).standard_normal(1000)
+    exact = scipy.sparse.linalg.spsolve(A.tocsc(), b)
+    rate = (np.sqrt(401.0) - 1.0) / (np.sqrt(401.0) + 1.0)
+    for timed in (False, True):
+        s = neon_amd.conjugate_gradient_hip(1e-30, limit, criterion=neon_amd.STOP_RELATIVE, context=ctx)
+        x = np.zeros(1000)
+        ctx.profile(timed)
+        try:
+            with pytest.raises(neon_amd.computational_error) as e:
+                s.solve(A, x, b)
+        finally:
+            ctx.profile(False)
+        assert (e.value.code, s.iterations) == (_capi.NEON_NONCONVERGED, limit)
+        d = x - exact
+        assert np.sqrt(d @ (A @ d)) <= 2.0 * rate ** limit * np.sqrt(exact @ b)
 
 
 @pytest.mark.parametrize("criterion", [neon_amd.STOP_RELATIVE, neon_amd.STOP_ABSOLUTE_PRECONDITIONED])
