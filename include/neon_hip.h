@@ -230,7 +230,7 @@ int neon_mesh_solve(neon_context* ctx, int solver, int criterion, double toleran
  * reference: a tuning knob; every shape gives the same products up to rounding (the order of
  * the row sums, and with NEON_SPMV_SYMMETRIC each lower block taken as the transpose of the
  * stored upper one). */
-#define NEON_SPMV_NONTEMPORAL 1 /* stream the values with nontemporal loads */
+#define NEON_SPMV_NONTEMPORAL 1 /* stream the values with nontemporal loads (a full sliced copy: from 240 MiB on) */
 #define NEON_SPMV_SLICED 256    /* the sliced copy of the values */
 #define NEON_SPMV_INDEX32 1024  /* with NEON_SPMV_SLICED: 32-bit per-lane column offsets even where
                                    16 bits fit (the default uses 16 bits when every offset fits) */

@@ -1828,6 +1828,7 @@ void device_mesh::attach_sliced(linear_operator& A, int precision, bool index32)
     }
     A.sell = true;
     A.sym = false;
+    if (vals * (precision == NEON_PRECISION_FP64 ? 8 : 4) <= kStreamedCopy) A.nb_nt = false;
     A.slices = slices_;
     A.sell_steps = max_degree_;
     A.sell_mean = double(sell_steps_) / slices_;

@@ -332,6 +332,17 @@ struct spmv_config
 constexpr int64_t kStageElements = int64_t(1) << 15;
 struct qp_state; // element_kernels.hpp
 
+// A sliced copy of at most this many bytes (a little under the 256 MB memory-side cache, which holds the
+// vectors too) is read with plain loads, a larger one with nontemporal loads if the flags ask for
+// them.  A solver reads the copy again in each iteration; nontemporal loads leave it in no L2, and
+// whether the next cache holds it then depends on what else was there: after a staged assembly,
+// whose blocks stay in the L2s, 14.4 us became 20.2 per FP32 product at 14^3 cells, 19.1 became 24.5 at
+// 15^3.  Nontemporal against plain, us per product: FP32 copies of 3.3, 9, 67, 221, 267, 378, 887 MB
+// 20.2 / 14.4, 23.3 / 15.3, 30.7 / 24.2, 45.4 / 39.9, 51.9 / 52.6, 87.6 / 92.4, 163.7 / 185.4; FP64
+// copies of 18, 134, 229, 360, 534, 1,774 MB 27.2 / 16.4, 37.3 / 28.1, 46.3 / 38.8, 81.1 / 80.3, 113.1 /
+// 116.5, 340.8 / 358.7.
+constexpr size_t kStreamedCopy = size_t(240) << 20;
+
 // Device-resident mesh: geometry, constitutive state, pattern, tangent and f_int.
 class device_mesh
 {

@@ -134,13 +134,13 @@ int neon_mesh_spmv_bench(neon_context* ctx, int32_t precision, int32_t lanes, in
             throw status_error(NEON_BAD_ARGUMENT, "bad SpMV flags");
         linear_operator A = m.op(precision);
         A.nb_lanes = lanes;
-        A.nb_nt = (flags & NEON_SPMV_NONTEMPORAL) != 0;
         A.blocks_override = blocks;
         A.sell = A.sym = false;
         if ((flags & NEON_SPMV_SLICED) && (flags & NEON_SPMV_SYMMETRIC) && m.symmetric_usable())
             m.attach_symmetric(A, precision);
         else if (flags & NEON_SPMV_SLICED)
             m.attach_sliced(A, precision, (flags & NEON_SPMV_INDEX32) != 0);
+        A.nb_nt = (flags & NEON_SPMV_NONTEMPORAL) != 0; // as asked, at every size
         int64_t const n = m.dofs();
         hipStream_t const s = ctx->stream;
         // NEON_MEASURE_DOT: the solvers' form with partials of x.y; NEON_MEASURE_DIRTY: each
@@ -192,13 +192,13 @@ int neon_mesh_spmv_apply(neon_context* ctx, int32_t precision, int32_t lanes, in
             throw status_error(NEON_BAD_ARGUMENT, "bad SpMV flags");
         linear_operator A = m.op(precision);
         A.nb_lanes = lanes;
-        A.nb_nt = (flags & NEON_SPMV_NONTEMPORAL) != 0;
         A.blocks_override = blocks;
         A.sell = A.sym = false;
         if ((flags & NEON_SPMV_SLICED) && (flags & NEON_SPMV_SYMMETRIC) && m.symmetric_usable())
             m.attach_symmetric(A, precision);
         else if (flags & NEON_SPMV_SLICED)
             m.attach_sliced(A, precision, (flags & NEON_SPMV_INDEX32) != 0);
+        A.nb_nt = (flags & NEON_SPMV_NONTEMPORAL) != 0; // as asked, at every size
         int64_t const n = m.dofs();
         hipStream_t const s = ctx->stream;
         device_array<double> xd, yd, part;

@@ -273,6 +273,32 @@ def test_mixed_cg_vector_part(ctx, dims):
     assert its <= 1.25 * its64 + 8, (its, its64)
 
 
+def test_a_small_full_copy_is_read_through_the_caches(ctx):
+    """The mixed loop's FP32 product on a full copy of 3 MB (boundary-first numbering), right after the
+    assembly: the default flags, which ask for nontemporal loads, must not make it slower than plain
+    loads do (they did by 40 %).  Least of five alternating runs; 20 % for the scatter of runs.  The
+    loads' kind does not change the solution."""
+    mg, b = _mesh(ctx, (14, 14, 14), "boundary", 0.0)
+    fixed = np.flatnonzero(b == 0.0).astype(np.int32)
+    plain = neon_amd.SPMV_SLICED | neon_amd.SPMV_SYMMETRIC
+    best, x = {}, {}
+    for _ in range(5):
+        for flags in (plain | neon_amd.SPMV_NONTEMPORAL, plain):
+            mg.spmv_config(flags=flags)
+            mg.assemble(neon_amd.PRECISION_MIXED)
+            mg.enforce_dirichlet(fixed, b.copy())
+            ctx.profile(True)
+            try:
+                x[flags] = mg.solve(b, tol=1e-10)[0]
+                count, ms = ctx.profile_read(_capi.KERNEL_SPMV_FP32)
+            finally:
+                ctx.profile(False)
+            best[flags] = min(best.get(flags, np.inf), ms / count)
+    print(best, flush=True)
+    assert np.array_equal(x[plain], x[plain | neon_amd.SPMV_NONTEMPORAL])
+    assert best[plain | neon_amd.SPMV_NONTEMPORAL] <= 1.2 * best[plain]
+
+
 def test_two_contexts_share_the_gpu():
     """Solves on two contexts from two threads at once: the grids take turns for the compute units."""
     import threading
