@@ -60,8 +60,9 @@ int lanes_for(double avg)
 // ---- the allocation-free CSR solve (neon_krylov_solve_csr_noalloc)
 // Its device memory beyond the caller's inputs and outputs lives in `scratch`, one copy per
 // GPU, held until the process ends: a validation flag, then the Jacobi inverse and the
-// solver's work vectors (9 vectors of at most kNoAllocRows entries: minv and BiCGSTAB's eight;
-// CG uses minv and three).  Every call on a GPU shares that GPU's copy, so calls that overlap
+// solver's work vectors (9 vectors of at most kNoAllocRows entries: minv and eight more, which
+// BiCGSTAB's launch loop takes as they are; the launch loop of CG needs three of them, and the
+// resident grids publish to those they do not keep vectors in).  Every call on a GPU shares that GPU's copy, so calls that overlap
 // on one GPU race; each call rewrites what it reads (the flag is cleared by a kernel, the
 // vectors are initialised by the solvers).
 constexpr int64_t kNoAllocRows = int64_t(1) << 18;

@@ -225,6 +225,8 @@ void kernel_profiler::read(int cls, bool reset, int64_t* count, double* ms)
 }
 
 // ================================================================== engine
+std::atomic<int64_t> device_allocations{0};
+
 csr_space::csr_space()
 {
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&stage), kCsrStage));
@@ -247,6 +249,7 @@ krylov_engine::krylov_engine(hipStream_t s) : s_(s)
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_ring_), 4 * sizeof(krylov_state)));
     for (auto& e : ring_events_) NEON_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     NEON_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_scalar_), sizeof(double)));
+    grid_begin();
 }
 
 krylov_engine::~krylov_engine()

@@ -6,6 +6,7 @@
 #include "common.hpp"
 #include "neon_hip.h"
 
+#include <atomic>
 #include <cstdint>
 #include <memory>
 #include <string>
@@ -14,6 +15,9 @@
 namespace neon_amd
 {
 struct krylov_state;
+
+// device_array allocations of the process so far (a test holds the allocation-free solve to none)
+extern std::atomic<int64_t> device_allocations;
 
 template <typename T>
 class device_array
@@ -30,6 +34,7 @@ public:
         release();
         if (n)
         {
+            ++device_allocations;
             hipError_t const e = hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T));
             if (e != hipSuccess)
             {

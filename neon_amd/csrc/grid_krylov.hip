@@ -206,9 +206,10 @@ bool shape_of(grid_shape& g, linear_operator const& A, int units, vector_need ne
 }
 } // namespace
 
+// What the resident grids need beyond a solve's own vectors: with the engine, so that a solve in
+// vectors of the caller's allocates nothing
 void krylov_engine::grid_begin()
 {
-    if (grid_units_) return;
     NEON_CHECK_HIP(hipGetDevice(&grid_device_));
     int units = 0;
     NEON_CHECK_HIP(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, grid_device_));
@@ -264,7 +265,6 @@ bool krylov_engine::grid_run(Batch&& batch)
 
 int krylov_engine::vector_blocks(int64_t n, int width)
 {
-    grid_begin();
     if (!grid_units_) return 0;
     // at least one 16-byte group per thread, a multiple of 8 (the XCDs' shares) from 8 on
     int64_t const b = std::min<int64_t>((n + int64_t(kVectorThreads) * width - 1) / (int64_t(kVectorThreads) * width),
@@ -300,7 +300,6 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
                               double tol, int32_t max_it, const krylov_work* work, solve_result& out)
 {
     if (prof && prof->enabled) return false; // per-launch timing needs the launches
-    grid_begin();
     if (!grid_units_ || A.blocks_override > 0) return false;
     grid_shape g;
     if (!shape_of(g, A, grid_units_, kCgNeed)) return false;
@@ -382,7 +381,6 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
                                     solve_result& out)
 {
     if (prof && prof->enabled) return false;
-    grid_begin();
     if (!grid_units_ || A.blocks_override > 0) return false;
     grid_shape g;
     if (!shape_of(g, A, grid_units_, kBicgNeed)) return false;

@@ -266,6 +266,17 @@ int neon_stream_probe(neon_context* ctx, int64_t bytes, int32_t reps, double* re
     });
 }
 
+// The process's device_array allocations so far.  Not a probe and not in the header: the test of the
+// allocation-free solve reads it.
+int neon_test_device_allocations(neon_context* ctx, int64_t* count)
+{
+    return measured(ctx, [&] {
+        if (!count) throw status_error(NEON_BAD_ARGUMENT, "null count");
+        *count = device_allocations;
+        return NEON_OK;
+    });
+}
+
 // How long the workgroups of a solver's resident grid wait for each other before the solve falls
 // back to launches (ticks of 10 ns; 0: a wait that has to wait at all gives up).  Not a probe and not
 // in the header: the fallback's test sets it.

@@ -132,6 +132,38 @@ def test_noalloc_solve_equals_allocating_solve(ctx, solver, criterion, unsym):
             assert np.linalg.norm(b - A @ x1) <= 1e-6 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("solver,unsym", [(_capi.SOLVER_CG, False), (_capi.SOLVER_BICGSTAB, True)])
+def test_noalloc_solve_allocates_nothing_on_a_fresh_context(solver, unsym):
+    """The first solve of a context does not move the library's count of its device allocations
+    (systems of one workgroup and of several, at the scratch's limit)."""
+    count = _capi.measure_lib().neon_test_device_allocations
+    count.restype, count.argtypes = C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]
+
+    def counted(ctx):
+        n = C.c_int64(0)
+        ctx.check(count(ctx.handle, C.byref(n)))
+        return n.value
+
+    for m in (4, 20, 64):
+        A, b = _system(m, unsym, 5)
+        n = A.shape[0]
+        c, dev = neon_amd.Context(0), _Device()
+        try:
+            rp, ci = dev.put(A.indptr.astype(np.int32)), dev.put(A.indices.astype(np.int32))
+            v, bd, xd = dev.put(A.data.astype(np.float64)), dev.put(b), dev.put(np.full(n, np.nan))
+            its, err = C.c_int32(0), C.c_double(0)
+            before = counted(c)
+            code = _noalloc()(c.handle, solver, _capi.STOP_RELATIVE, n, int(A.indptr[-1]), rp, ci, v, bd, xd, 1e-10,
+                              20000, C.byref(its), C.byref(err))
+            after = counted(c)
+            c.check(code)
+            assert after == before, (m, before, after)
+            assert np.linalg.norm(b - A @ dev.get(xd, b)) <= 1e-6 * np.linalg.norm(b)
+        finally:
+            dev.release()
+            c.close()
+
+
 def test_noalloc_refuses_what_does_not_fit(ctx):
     fn = _noalloc()
     its, err = C.c_int32(0), C.c_double(0)
