@@ -405,6 +405,7 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
         cg_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, criterion, tol, max_it);
         NEON_CHECK_HIP(hipGetLastError());
         auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        auto const since = grid_clock::now();
         launched = 0;
         linear_operator Ak = A; // its products alternate in order
         run_batches(st, launched, [&] {
@@ -427,7 +428,7 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
                                                            criterion, tol, max_it);
             }
         });
-        if (!vb || !vector_gave_up()) break;
+        if (!vb || !vector_gave_up(since)) break;
         if (prof) prof->discard();
     }
     res = finish_solve(*host_state_, criterion);
@@ -633,6 +634,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     for (int vb = scaled ? vector_blocks(n, 4) : 0;; vb = 0)
     {
         auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        auto const since = grid_clock::now();
         if (scaled)
             mixed_init_scaled_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv64_scaled, part_rr, part_rz);
         else
@@ -693,7 +695,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
                                                                         nxt, max_it);
             }
         });
-        if (!vb || !vector_gave_up()) break;
+        if (!vb || !vector_gave_up(since)) break;
         if (prof) prof->discard();
     }
     // fold whatever the recurrence holds since the last reliable update

@@ -6,7 +6,9 @@
 #include "common.hpp"
 #include "neon_hip.h"
 
+#include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <memory>
 #include <string>
@@ -247,7 +249,12 @@ public:
     int poll_every = 16;
     // ticks (100 MHz) that a resident grid's workgroups wait for each other before the solve falls
     // back to launches: another process may hold the compute units that some of them need
-    uint64_t grid_patience = 100ull * 1000 * 1000;
+    void set_grid_patience(uint64_t ticks)
+    {
+        grid_patience_ = ticks;
+        grid_rest_until_ = {};
+    }
+    int64_t grid_give_ups = 0;
     // reliable-update trigger of the mixed-precision CG: ||r32|| < delta ||r at last update||
 #ifndef NEON_RELIABLE_DELTA
 #define NEON_RELIABLE_DELTA 0.1
@@ -284,15 +291,29 @@ private:
     bool bicgstab64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion,
                          double tol, int32_t max_it, const krylov_work* work, solve_result& out);
     // an iteration's vector part in one launch (vector_iteration): the workgroups for n entries (0:
-    // not available) and the launches; after a loop with them, whether one gave up (the loop then
-    // runs again without them)
+    // not available) and the launches; vector_gave_up, after a loop with them that began at `since`:
+    // whether one gave up (the loop then runs again without them)
     int vector_blocks(int64_t n, int width);
     void cg_vector(int blocks, int64_t n, double* r, const double* Ap, const double* minv, double* x, double* p,
                    const double* part, int npart, const krylov_state* st, krylov_state* next, int criterion, double tol,
                    int32_t max_it);
     void mixed_vector(int blocks, int64_t n, float* r, const float* Ap, float* x, float* p, const double* part,
                       int npart, const krylov_state* st, krylov_state* next, int32_t max_it);
-    bool vector_gave_up();
+    // A grid that gave up cost its solve the patience and the work so far, and what kept it out is
+    // likely to be there for the next one too: solves take launches for kGridRest times as long as
+    // was lost (at least kGridRest times 10 ms), so that a lasting cause costs 1 / kGridRest.
+    static constexpr int kGridRest = 64;
+    using grid_clock = std::chrono::steady_clock;
+    bool grid_resting() const { return grid_clock::now() < grid_rest_until_; }
+    void grid_gave_up(grid_clock::time_point since)
+    {
+        auto const now = grid_clock::now();
+        grid_rest_until_ = now + kGridRest * std::max<grid_clock::duration>(now - since, std::chrono::milliseconds(10));
+        ++grid_give_ups;
+    }
+    grid_clock::time_point grid_rest_until_{};
+    uint64_t grid_patience_ = 100ull * 1000 * 1000;
+    bool vector_gave_up(grid_clock::time_point since);
     void grid_begin();
     void grid_clear();
     grid_link grid_next(uint32_t exchanges);

@@ -229,7 +229,7 @@ void krylov_engine::grid_clear()
 grid_link krylov_engine::grid_next(uint32_t exchanges)
 {
     if (grid_epoch_ > UINT32_MAX - exchanges - 1) grid_clear();
-    grid_link const l{grid_slots_.data(), state_.data() + 3, grid_patience, grid_epoch_};
+    grid_link const l{grid_slots_.data(), state_.data() + 3, grid_patience_, grid_epoch_};
     grid_epoch_ += exchanges;
     return l;
 }
@@ -241,6 +241,7 @@ grid_link krylov_engine::grid_next(uint32_t exchanges)
 template <typename Batch>
 bool krylov_engine::grid_run(Batch&& batch)
 {
+    auto const since = grid_clock::now();
     auto step = [&](bool first, int slot) {
         batch(first);
         NEON_CHECK_HIP(hipGetLastError());
@@ -260,12 +261,13 @@ bool krylov_engine::grid_run(Batch&& batch)
     if (!host_ring_[2 * wait + 1].done && host_state_->done != KRYLOV_ABORTED) return true;
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
     grid_clear();
+    grid_gave_up(since);
     return false;
 }
 
 int krylov_engine::vector_blocks(int64_t n, int width)
 {
-    if (!grid_units_) return 0;
+    if (!grid_units_ || grid_resting()) return 0;
     // at least one 16-byte group per thread, a multiple of 8 (the XCDs' shares) from 8 on
     int64_t const b = std::min<int64_t>((n + int64_t(kVectorThreads) * width - 1) / (int64_t(kVectorThreads) * width),
                                         std::min(grid_units_, kGridMaxBlocks));
@@ -287,12 +289,13 @@ void krylov_engine::mixed_vector(int blocks, int64_t n, float* r, const float* A
     mixed_vector_kernel<<<blocks, kVectorThreads, 0, s_>>>(n, r, Ap, x, p, part, npart, st, next, grid_next(1), max_it);
 }
 
-bool krylov_engine::vector_gave_up()
+bool krylov_engine::vector_gave_up(grid_clock::time_point since)
 {
     NEON_CHECK_HIP(hipMemcpyAsync(host_ring_, state_.data() + 3, sizeof(krylov_state), hipMemcpyDeviceToHost, s_));
     NEON_CHECK_HIP(hipStreamSynchronize(s_));
     if (!host_ring_[0].done) return false;
     grid_clear();
+    grid_gave_up(since);
     return true;
 }
 
@@ -300,7 +303,7 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
                               double tol, int32_t max_it, const krylov_work* work, solve_result& out)
 {
     if (prof && prof->enabled) return false; // per-launch timing needs the launches
-    if (!grid_units_ || A.blocks_override > 0) return false;
+    if (!grid_units_ || A.blocks_override > 0 || grid_resting()) return false;
     grid_shape g;
     if (!shape_of(g, A, grid_units_, kCgNeed)) return false;
 
@@ -381,7 +384,7 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
                                     solve_result& out)
 {
     if (prof && prof->enabled) return false;
-    if (!grid_units_ || A.blocks_override > 0) return false;
+    if (!grid_units_ || A.blocks_override > 0 || grid_resting()) return false;
     grid_shape g;
     if (!shape_of(g, A, grid_units_, kBicgNeed)) return false;
     int64_t const n = A.n;

@@ -284,7 +284,17 @@ int neon_test_grid_patience(neon_context* ctx, int64_t ticks)
 {
     return measured(ctx, [&] {
         if (ticks < 0) throw status_error(NEON_BAD_ARGUMENT, "negative patience");
-        ctx->engine->grid_patience = uint64_t(ticks);
+        ctx->engine->set_grid_patience(uint64_t(ticks));
+        return NEON_OK;
+    });
+}
+
+// How many resident grids of the context have given up (for the same test).
+int neon_test_grid_give_ups(neon_context* ctx, int64_t* count)
+{
+    return measured(ctx, [&] {
+        if (!count) throw status_error(NEON_BAD_ARGUMENT, "null count");
+        *count = ctx->engine->grid_give_ups;
         return NEON_OK;
     });
 }

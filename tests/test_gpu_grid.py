@@ -255,6 +255,57 @@ def test_a_grid_that_gives_up_is_solved_by_launches(ctx):
     assert np.array_equal(mixed()[0], patient[0])
 
 
+def test_a_grid_that_gave_up_rests(ctx):
+    """After a grid has given up, the context's solves take launches for a while (64 times what was
+    lost, at least 0.64 s) instead of each waiting again; then the grid is tried once more.  With
+    no patience every try gives up, so the count of give-ups is the count of tries.  A solve whose
+    grid gave up does not try the one-launch vector part either; the vector part of a system too
+    large for the grid, and of the mixed loop, gives up as the grid does."""
+    import time
+
+    lib = _capi.measure_lib()
+    patience, count = lib.neon_test_grid_patience, lib.neon_test_grid_give_ups
+    patience.restype, patience.argtypes = C.c_int, [C.c_void_p, C.c_int64]
+    count.restype, count.argtypes = C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]
+
+    def tries():
+        n = C.c_int64(0)
+        ctx.check(count(ctx.handle, C.byref(n)))
+        return n.value
+
+    A, b = _spd(40000, 20, 8)
+    big, bb = _spd(1300000, 4, 9)
+    mg, bm = _mesh(ctx, (30, 29, 31), "grid", 0.0)
+    mg.assemble(neon_amd.PRECISION_MIXED)
+    mg.enforce_dirichlet(problems.block_rollers(31, dims=(30, 29, 31)).fixed_dofs(), bm)
+    solve = lambda: _solve_csr(ctx, neon_amd.conjugate_gradient_hip, A, b)
+    solves = [lambda: _solve_csr(ctx, neon_amd.conjugate_gradient_hip, big, bb), lambda: mg.solve(bm, tol=1e-10)]
+    solve()  # the memory the context keeps
+    try:
+        ctx.check(patience(ctx.handle, 0))
+        start, first = time.perf_counter(), tries()
+        x = solve()[0]
+        done = 1
+        while time.perf_counter() - start < 0.3:
+            assert np.array_equal(solve()[0], x)
+            done += 1
+        assert done >= 5 and tries() == first + 1, (done, tries() - first)
+        time.sleep(1.0)
+        # the try before took less than 10 ms of waiting and work, or 64 times that is over by now
+        assert np.array_equal(solve()[0], x)
+        assert tries() <= first + 2
+        for other in solves:
+            ctx.check(patience(ctx.handle, 0))  # ends the rest
+            n = tries()
+            other()
+            assert tries() == n + 1
+            other()
+            assert tries() == n + 1
+    finally:
+        ctx.check(patience(ctx.handle, 10 ** 8))
+    assert np.linalg.norm(b - A @ x) <= 1.1e-10 * np.linalg.norm(b)
+
+
 # one workgroup, its last entries fewer than a 16-byte group; several; and more entries than the
 # threads keep in registers
 @pytest.mark.parametrize("dims", [(1, 1, 1), (7, 6, 5), (20, 19, 23), (44, 43, 45), (104, 102, 101)])
