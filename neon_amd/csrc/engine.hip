@@ -335,10 +335,11 @@ solve_result finish_solve(const krylov_state& s, int criterion)
 // Drives a device-resident Krylov loop: `batch` launches poll_every iterations (advancing
 // `launched`; the state after `launched` iterations is st[launched & 1]).  The host keeps one
 // batch queued ahead of the one whose final state it is waiting for, so the device never idles
-// on a poll; iterations launched after convergence are no-ops.  On return the stream is idle
+// on a poll; iterations launched after convergence are no-ops.  With `hold` (null: none) other
+// solves that wait for compute units get them between two batches.  On return the stream is idle
 // and host_state_ holds the final state.
 template <typename Batch>
-void krylov_engine::run_batches(krylov_state* st, int64_t& launched, Batch&& batch)
+void krylov_engine::run_batches(krylov_state* st, int64_t& launched, unit_hold* hold, Batch&& batch)
 {
     auto snapshot = [&](int slot) {
         NEON_CHECK_HIP(hipMemcpyAsync(host_ring_ + slot, st + (launched & 1), sizeof(krylov_state),
@@ -354,6 +355,12 @@ void krylov_engine::run_batches(krylov_state* st, int64_t& launched, Batch&& bat
         snapshot(1);
         for (int wait = 1;; wait ^= 1)
         {
+            if (hold && hold->wanted())
+            {
+                NEON_CHECK_HIP(hipEventSynchronize(ring_events_[wait]));
+                if (host_ring_[wait].done) break;
+                hold->yield();
+            }
             batch();
             NEON_CHECK_HIP(hipGetLastError());
             snapshot(wait ^ 1);
@@ -404,11 +411,11 @@ solve_result krylov_engine::cg64(const linear_operator& A, const double* b, doub
         cg_init_kernel<<<nb, kBlock, 0, s_>>>(n, x, r, p, b, minv, part_rr, part_rz);
         cg_init_state_kernel<<<1, kBlock, 0, s_>>>(part_rr, part_rz, nb, st, criterion, tol, max_it);
         NEON_CHECK_HIP(hipGetLastError());
-        auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        auto const hold = vb ? std::make_unique<unit_hold>(grid_device_, vb, grid_units_) : nullptr;
         auto const since = grid_clock::now();
         launched = 0;
         linear_operator Ak = A; // its products alternate in order
-        run_batches(st, launched, [&] {
+        run_batches(st, launched, hold.get(), [&] {
             for (int k = 0; k < poll_every; ++k, ++launched)
             {
                 krylov_state* cur = st + (launched & 1);
@@ -516,7 +523,7 @@ solve_result krylov_engine::bicgstab64(const linear_operator& A, const double* b
     // the state is a single slot (decision kernels write it between the grid kernels that read
     // it), so run_batches reads st[launched & 1] = st[0] with launched kept even
     int64_t launched = 0;
-    run_batches(st, launched, [&] {
+    run_batches(st, launched, nullptr, [&] {
         for (int k = 0; k < poll_every; ++k)
         {
             if (!cuda_rule)
@@ -633,7 +640,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     int64_t launched = 0;
     for (int vb = scaled ? vector_blocks(n, 4) : 0;; vb = 0)
     {
-        auto const hold = vb ? hold_units(grid_device_, vb, grid_units_) : nullptr;
+        auto const hold = vb ? std::make_unique<unit_hold>(grid_device_, vb, grid_units_) : nullptr;
         auto const since = grid_clock::now();
         if (scaled)
             mixed_init_scaled_kernel<<<nb, kBlock, 0, s_>>>(n, b, x, r32, x32, p32, minv64_scaled, part_rr, part_rz);
@@ -646,7 +653,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
         linear_operator Ar = A;
         if (Ar.node_block && (Ar.sell || Ar.sym)) Ar.blocks_override = 2048;
         launched = 0;
-        run_batches(st, launched, [&] {
+        run_batches(st, launched, hold.get(), [&] {
             for (int k = 0; k < poll_every; ++k, ++launched)
             {
                 krylov_state* cur = st + (launched & 1);

@@ -205,8 +205,24 @@ struct csr_space
     csr_space& operator=(csr_space const&) = delete;
 };
 
-class unit_hold; // grid_krylov.hip: compute units held for a resident grid
-std::shared_ptr<unit_hold> hold_units(int device, int count, int units);
+// Compute units of a GPU held for one solve's resident grids (grid_krylov.hip).  A solve with nothing
+// in flight lets others have their turn with yield() while wanted(): it holds them for a batch of
+// iterations at a time if another solve waits, for all of them otherwise.
+class unit_pool;
+class unit_hold
+{
+public:
+    unit_hold(int device, int count, int units);
+    ~unit_hold();
+    unit_hold(unit_hold const&) = delete;
+    unit_hold& operator=(unit_hold const&) = delete;
+    bool wanted() const;
+    void yield();
+
+private:
+    unit_pool& pool_;
+    int count_, units_;
+};
 
 class krylov_engine
 {
@@ -283,7 +299,7 @@ private:
     krylov_state* host_ring_ = nullptr;
     hipEvent_t ring_events_[2] = {nullptr, nullptr};
     template <typename Batch>
-    void run_batches(krylov_state* st, int64_t& launched, Batch&& batch);
+    void run_batches(krylov_state* st, int64_t& launched, unit_hold* hold, Batch&& batch);
     // resident-grid loops (grid_krylov.hip): false when the solve does not qualify or its grid
     // gave up; the launch-per-phase loop then solves
     bool cg64_grid(const linear_operator& A, const double* b, double* x, const double* minv, int criterion, double tol,
@@ -318,7 +334,7 @@ private:
     void grid_clear();
     grid_link grid_next(uint32_t exchanges);
     template <typename Batch>
-    bool grid_run(Batch&& batch);
+    bool grid_run(unit_hold& hold, Batch&& batch);
     int grid_device_ = 0, grid_units_ = 0;
     uint32_t grid_epoch_ = 1;
     device_array<uint64_t> grid_slots_;

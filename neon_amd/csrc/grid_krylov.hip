@@ -4,8 +4,8 @@
 #include "grid_kernels.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
-#include <memory>
 #include <mutex>
 
 namespace neon_amd
@@ -44,10 +44,11 @@ __global__ __launch_bounds__(kVectorThreads) void mixed_vector_kernel(int64_t n,
 namespace
 {
 constexpr int64_t kGridLds = 160 * 1024 - 1024; // LDS of a compute unit less the static arrays
+} // namespace
 
 // Compute units of each GPU that this process's resident grids may still take.  A grid's
 // workgroups wait for each other, so two grids that together exceed the GPU must not be in flight at
-// once; a solve waits here until the ones before it have left enough room.
+// once; a solve waits here until the ones before it have left enough room, in the order of arrival.
 class unit_pool
 {
 public:
@@ -59,9 +60,14 @@ public:
     static constexpr int kDevices = 64;
     void take(int want, int units)
     {
-        std::unique_lock<std::mutex> lock(m_);
-        cv_.wait(lock, [&] { return used_ + want <= units; });
-        used_ += want;
+        {
+            std::unique_lock<std::mutex> lock(m_);
+            uint64_t const ticket = arrived_++;
+            cv_.wait(lock, [&] { return served_ == ticket && used_ + want <= units; });
+            ++served_;
+            used_ += want;
+        }
+        cv_.notify_all(); // the next in the queue may fit too
     }
     void give(int count)
     {
@@ -71,32 +77,25 @@ public:
         }
         cv_.notify_all();
     }
+    bool waited_for() const { return arrived_ != served_; }
 
 private:
     std::mutex m_;
     std::condition_variable cv_;
     int used_ = 0;
+    std::atomic<uint64_t> arrived_{0}, served_{0};
 };
 
-
-} // namespace
-
-class unit_hold
+unit_hold::unit_hold(int device, int count, int units) : pool_(unit_pool::of(device)), count_(count), units_(units)
 {
-public:
-    unit_hold(int device, int want, int units) : pool_(unit_pool::of(device)), count_(want) { pool_.take(want, units); }
-    ~unit_hold() { pool_.give(count_); }
-    unit_hold(unit_hold const&) = delete;
-    unit_hold& operator=(unit_hold const&) = delete;
-
-private:
-    unit_pool& pool_;
-    int count_;
-};
-
-std::shared_ptr<unit_hold> hold_units(int device, int count, int units)
+    pool_.take(count_, units_);
+}
+unit_hold::~unit_hold() { pool_.give(count_); }
+bool unit_hold::wanted() const { return pool_.waited_for(); }
+void unit_hold::yield()
 {
-    return std::make_shared<unit_hold>(device, count, units);
+    pool_.give(count_);
+    pool_.take(count_, units_);
 }
 
 namespace
@@ -239,7 +238,7 @@ grid_link krylov_engine::grid_next(uint32_t exchanges)
 // end return at once).  host_state_ holds the final state; false when the grid gave up (the
 // state and vectors are then worthless).
 template <typename Batch>
-bool krylov_engine::grid_run(Batch&& batch)
+bool krylov_engine::grid_run(unit_hold& hold, Batch&& batch)
 {
     auto const since = grid_clock::now();
     auto step = [&](bool first, int slot) {
@@ -253,6 +252,13 @@ bool krylov_engine::grid_run(Batch&& batch)
     int wait = 0;
     for (;; wait ^= 1)
     {
+        if (hold.wanted())
+        {
+            // another solve's turn, once the launch in flight is through
+            NEON_CHECK_HIP(hipEventSynchronize(ring_events_[wait]));
+            if (host_ring_[2 * wait].done || host_ring_[2 * wait + 1].done) break;
+            hold.yield();
+        }
         step(false, wait ^ 1);
         NEON_CHECK_HIP(hipEventSynchronize(ring_events_[wait]));
         if (host_ring_[2 * wait].done || host_ring_[2 * wait + 1].done) break;
@@ -330,10 +336,10 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
     int const iters = int(std::min<int64_t>(few ? buffers / 2 : buffers, 64));
     if (iters < 1) return false;
     krylov_state* st = state_.data() + 2;
-    auto const hold = hold_units(grid_device_, g.blocks, grid_units_);
+    unit_hold hold(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto kernel, auto rows) {
         allow_lds(kernel, g.lds);
-        return grid_run([&, kernel](bool first) {
+        return grid_run(hold, [&, kernel](bool first) {
             kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, first ? b : nullptr, x, r, minv,
                                                                   st, grid_next(uint32_t(3 * iters + 2)), iters,
                                                                   criterion, tol, max_it);
@@ -409,11 +415,11 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
     if (iters < 1) return false;
     int const cuda_rule = criterion == NEON_STOP_ABSOLUTE_PRECONDITIONED ? 1 : 0;
     krylov_state* st = state_.data() + 2;
-    auto const hold = hold_units(grid_device_, g.blocks, grid_units_);
+    unit_hold hold(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto rows) {
         auto kernel = bicg_grid_kernel<decltype(rows)>;
         allow_lds(kernel, g.lds);
-        return grid_run([&, kernel](bool first) {
+        return grid_run(hold, [&, kernel](bool first) {
             kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, b, x, r, r0, p, v, minv, st,
                                                                   grid_next(uint32_t(7 * iters + 1)), first ? 1 : 0,
                                                                   iters, cuda_rule, tol, max_it);

@@ -375,6 +375,52 @@ def test_two_contexts_share_the_gpu():
         assert np.array_equal(results[k][0], results[k][1]) and np.array_equal(results[k][0], results[k][2])
 
 
+# a large solve in the launch loop with its one-launch vector part (mixed, FP64) and in the resident grid,
+# each a good part of a second long (none reaches its tolerance)
+@pytest.mark.parametrize("dims,precision,tol,limit", [((104, 102, 101), "mixed", 1e-30, 6000),
+                                                      ((104, 102, 101), "fp64", 1e-30, 3000),
+                                                      ((52, 50, 51), "fp64", 1e-150, 8000)])
+def test_a_small_solve_takes_turns_with_a_large_one(ctx, dims, precision, tol, limit):
+    """Small solves in one thread while a large one, which holds every compute unit, runs in another:
+    they get their turn between the large one's batches (2 to 3 ms each; a small solve here takes
+    some ten turns) instead of waiting for its end, and neither's result changes."""
+    import threading
+
+    print(dims, precision, flush=True)
+    large = neon_amd.Context(0)
+    try:
+        mg, b = _mesh(large, dims, "grid", 0.0)
+        if precision == "mixed":
+            mg.assemble(neon_amd.PRECISION_MIXED)
+            mg.enforce_dirichlet(problems.block_rollers(max(dims), dims=dims).fixed_dofs(), b)
+        small, c = _mesh(ctx, (9, 8, 7), "grid", 0.0)
+        out = {}
+
+        def solve_large(key):
+            try:
+                mg.solve(b, tol=tol, max_iterations=limit)
+            except neon_amd.computational_error as e:
+                out[key] = e.code
+            out[key, "u"] = mg.solve(b, tol=1e-6)[0]
+
+        alone = small.solve(c, tol=1e-10)[0]
+        solve_large("alone")
+        thread = threading.Thread(target=solve_large, args=("shared",))
+        thread.start()
+        count = 0
+        while thread.is_alive():
+            assert np.array_equal(small.solve(c, tol=1e-10)[0], alone)
+            count += 1
+        thread.join()
+        print(count, "small solves", flush=True)
+        assert out["alone"] == out["shared"] == _capi.NEON_NONCONVERGED
+        assert np.array_equal(out["alone", "u"], out["shared", "u"])
+        assert count >= 6, count
+        del mg
+    finally:
+        large.close()
+
+
 def _unsymmetric(n, per_row, seed):
     A, b = _spd(n, per_row, seed)
     rng = np.random.default_rng(seed + 1)
