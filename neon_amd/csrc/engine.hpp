@@ -271,6 +271,8 @@ public:
         grid_rest_until_ = {};
     }
     int64_t grid_give_ups = 0;
+    // the number of the next exchange (unique among those whose words the slots may still hold)
+    uint32_t grid_epoch = 1;
     // reliable-update trigger of the mixed-precision CG: ||r32|| < delta ||r at last update||
 #ifndef NEON_RELIABLE_DELTA
 #define NEON_RELIABLE_DELTA 0.1
@@ -336,7 +338,6 @@ private:
     template <typename Batch>
     bool grid_run(unit_hold& hold, Batch&& batch);
     int grid_device_ = 0, grid_units_ = 0;
-    uint32_t grid_epoch_ = 1;
     device_array<uint64_t> grid_slots_;
     device_array<double> grid_ring_, grid_r_, grid_bicg_;
     double* host_scalar_ = nullptr;

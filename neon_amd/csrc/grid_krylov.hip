@@ -221,15 +221,20 @@ void krylov_engine::grid_clear()
 {
     fill_zero(s_, int64_t(grid_slots_.size()), reinterpret_cast<double*>(grid_slots_.data()));
     fill_zero(s_, 2 * sizeof(krylov_state) / sizeof(double), reinterpret_cast<double*>(state_.data() + 2));
-    grid_epoch_ = 1;
+    grid_epoch = 1;
 }
 
 // The link for one launch of at most `exchanges` exchanges
 grid_link krylov_engine::grid_next(uint32_t exchanges)
 {
-    if (grid_epoch_ > UINT32_MAX - exchanges - 1) grid_clear();
-    grid_link const l{grid_slots_.data(), state_.data() + 3, grid_patience_, grid_epoch_};
-    grid_epoch_ += exchanges;
+    if (grid_epoch > UINT32_MAX - exchanges - 1)
+    {
+        // the numbers start again: no slot may hold one of them (the solve's state stays)
+        fill_zero(s_, int64_t(grid_slots_.size()), reinterpret_cast<double*>(grid_slots_.data()));
+        grid_epoch = 1;
+    }
+    grid_link const l{grid_slots_.data(), state_.data() + 3, grid_patience_, grid_epoch};
+    grid_epoch += exchanges;
     return l;
 }
 

@@ -299,4 +299,14 @@ int neon_test_grid_give_ups(neon_context* ctx, int64_t* count)
     });
 }
 
+// Sets the number of the resident grids' next exchange (for the test of its wrap).
+int neon_test_grid_epoch(neon_context* ctx, uint32_t epoch)
+{
+    return measured(ctx, [&] {
+        if (epoch < ctx->engine->grid_epoch) throw status_error(NEON_BAD_ARGUMENT, "exchange numbers only rise");
+        ctx->engine->grid_epoch = epoch;
+        return NEON_OK;
+    });
+}
+
 } // extern "C"

@@ -306,6 +306,43 @@ def test_a_grid_that_gave_up_rests(ctx):
     assert np.linalg.norm(b - A @ x) <= 1.1e-10 * np.linalg.norm(b)
 
 
+# numbers left for a first launch and not for the second; and for none
+@pytest.mark.parametrize("left", [300, 1])
+def test_the_exchange_numbers_start_again(left):
+    """A context's exchanges are numbered in 32 bits.  Where the numbers run out the slots are cleared
+    and the numbers start again at 1, in the middle of a solve too: every result has the bits it
+    has on a fresh context, CG (grid, small grid and the launch loop's vector part) and BiCGSTAB."""
+    set_number = _capi.measure_lib().neon_test_grid_epoch
+    set_number.restype, set_number.argtypes = C.c_int, [C.c_void_p, C.c_uint32]
+    A, b = _spd(40000, 20, 8)
+    U, ub = _unsymmetric(20000, 30, 6)
+    lap = _laplacian(120)
+    cg, bi = neon_amd.conjugate_gradient_hip, neon_amd.biconjugate_gradient_stabilised_hip
+    out = {}
+    for key in ("fresh", "wrapped"):
+        c = neon_amd.Context(0)
+        try:
+            mg, bm = _mesh(c, (20, 21, 19), "grid", 0.0)
+            solves = [lambda: _solve_csr(c, cg, A, b), lambda: _solve_csr(c, cg, lap, np.ones(14400)),
+                      lambda: _solve_csr(c, bi, U, ub), lambda: mg.solve(bm, tol=1e-10)]
+            results = []
+            for solve in solves:
+                if key == "wrapped":
+                    c.check(set_number(c.handle, 2 ** 32 - 1 - left))
+                results.append(solve())
+            mg.assemble(neon_amd.PRECISION_MIXED)
+            mg.enforce_dirichlet(problems.block_rollers(21, dims=(20, 21, 19)).fixed_dofs(), bm.copy())
+            if key == "wrapped":
+                c.check(set_number(c.handle, 2 ** 32 - 1 - min(left, 20)))
+            results.append(mg.solve(bm, tol=1e-10))
+            out[key] = results
+            del mg
+        finally:
+            c.close()
+    for fresh, wrapped in zip(out["fresh"], out["wrapped"]):
+        assert np.array_equal(fresh[0], wrapped[0]) and fresh[1] == wrapped[1]
+
+
 # one workgroup, its last entries fewer than a 16-byte group; several; and more entries than the
 # threads keep in registers
 @pytest.mark.parametrize("dims", [(1, 1, 1), (7, 6, 5), (20, 19, 23), (44, 43, 45), (104, 102, 101)])
