@@ -3,6 +3,7 @@
 // point returns NEON_NO_DEVICE.
 #include "engine.hpp"
 #include "newton.hpp"
+#include "spmv_layouts.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -59,7 +60,7 @@ int lanes_for(double avg)
 
 // ---- the allocation-free CSR solve (neon_krylov_solve_csr_noalloc)
 // Its device memory beyond the caller's inputs and outputs lives in `scratch`, one copy per
-// GPU, held until the process ends: a validation flag, then the Jacobi inverse and the
+// GPU, held until the process ends: the checks' flags, then the Jacobi inverse and the
 // solver's work vectors (9 vectors of at most kNoAllocRows entries: minv and eight more, which
 // BiCGSTAB's launch loop takes as they are; the launch loop of CG needs three of them, and the
 // resident grids publish to those they do not keep vectors in).  Every call on a GPU shares that GPU's copy, so calls that overlap
@@ -91,12 +92,13 @@ double* scratch_address(int device)
     return scratch_ptr[device];
 }
 
+// flag[0]: the check's verdict; flag[1], as an unsigned integer: the longest row
 __global__ void clear_flag_kernel(double* flag)
 {
-    if (threadIdx.x == 0) flag[0] = 0.0;
+    if (threadIdx.x < 2) flag[threadIdx.x] = 0.0;
 }
 
-// flag <- 1 if the CSR arrays are malformed: row_ptr[0] != 0, row_ptr[n] != nnz, a decreasing
+// flag[0] <- 1 if the CSR arrays are malformed: row_ptr[0] != 0, row_ptr[n] != nnz, a decreasing
 // row pointer or a column outside [0, n).  Reads row_ptr[0..n] and col[0..nnz) only.
 __global__ void check_csr_kernel(int32_t n, int64_t nnz, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
                                  double* flag)
@@ -104,10 +106,54 @@ __global__ void check_csr_kernel(int32_t n, int64_t nnz, const int32_t* __restri
     int64_t const stride = int64_t(gridDim.x) * blockDim.x;
     int64_t const t0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     bool bad = false;
+    int32_t longest = 0;
     if (t0 == 0) bad = rp[0] != 0 || int64_t(rp[n]) != nnz;
-    for (int64_t r = t0; r < n; r += stride) bad = bad || rp[r + 1] < rp[r];
+    for (int64_t r = t0; r < n; r += stride)
+    {
+        bad = bad || rp[r + 1] < rp[r];
+        longest = max(longest, rp[r + 1] - rp[r]);
+    }
     for (int64_t q = t0; q < nnz; q += stride) bad = bad || ci[q] < 0 || ci[q] >= n;
     if (bad) flag[0] = 1.0;
+    for (int m = 32; m > 0; m >>= 1) longest = max(longest, __shfl_xor(longest, m, 64));
+    if ((threadIdx.x & 63) == 0 && longest > 0)
+        atomicMax(reinterpret_cast<unsigned long long*>(flag + 1), (unsigned long long)longest);
+}
+
+// After check_csr_kernel: flag[0] <- 2 if the arrays are sound but their rows too unequal for the resident
+// grid, whose workgroups take `rows` rows each (at most 256 of them)
+__global__ __launch_bounds__(256) void csr_evenness_kernel(int32_t n, int64_t nnz, int64_t rows, int lanes,
+                                                           const int32_t* __restrict__ rp, double* flag)
+{
+    __shared__ int64_t largest[256];
+    int const t = threadIdx.x;
+    int64_t const blocks = (n + rows - 1) / rows;
+    int64_t most = 0;
+    for (int64_t k = t; k < blocks; k += 256)
+    {
+        int64_t const end = (k + 1) * rows < n ? (k + 1) * rows : n;
+        most = max(most, int64_t(rp[end]) - rp[k * rows]);
+    }
+    largest[t] = most;
+    __syncthreads();
+    if (t != 0 || flag[0] != 0.0) return;
+    for (int k = 1; k < 256; ++k) most = max(most, largest[k]);
+    int64_t const longest = int64_t(*reinterpret_cast<const unsigned long long*>(flag + 1));
+    if (!csr_grid_pays(most, double(nnz) / double(blocks), longest, lanes)) flag[0] = 2.0;
+}
+
+// The same for arrays in host memory (sound ones)
+bool csr_is_uneven(int32_t n, int64_t nnz, int64_t rows, int lanes, const int32_t* row_ptr)
+{
+    int64_t const blocks = (n + rows - 1) / rows;
+    double const mean = double(nnz) / double(blocks);
+    int64_t most = 0;
+    for (int64_t k = 0; k < blocks; ++k)
+        most = std::max<int64_t>(most, int64_t(row_ptr[std::min<int64_t>((k + 1) * rows, n)]) - row_ptr[k * rows]);
+    if (csr_grid_pays(most, mean, 0, lanes)) return false;
+    int32_t longest = 0;
+    for (int32_t r = 0; r < n; ++r) longest = std::max(longest, row_ptr[r + 1] - row_ptr[r]);
+    return !csr_grid_pays(most, mean, longest, lanes);
 }
 } // namespace
 
@@ -214,7 +260,7 @@ int neon_krylov_solve_csr(neon_context* ctx, int solver, int criterion, int prec
         size_t const n_ = size_t(n), z = size_t(std::max<int64_t>(nnz, 1));
         size_t const at_v = place(z * 8), at_b = place(n_ * 8), at_rp = place((n_ + 1) * 4), at_ci = place(z * 4);
         size_t const up = end;
-        size_t const at_x = place(n_ * 8), at_m = place(n_ * 8), at_flag = place(8);
+        size_t const at_x = place(n_ * 8), at_m = place(n_ * 8), at_flag = place(16);
         size_t const at_v32 = place(precision == NEON_PRECISION_FP64 ? 0 : z * 4);
         space.dev.reserve(end);
         unsigned char* const dev = space.dev.data();
@@ -269,6 +315,7 @@ int neon_krylov_solve_csr(neon_context* ctx, int solver, int criterion, int prec
         A.rp = drp;
         A.ci = dci;
         A.lanes_per_row = lanes_for(double(nnz) / n);
+        A.uneven = csr_is_uneven(n, nnz, k.csr_block_rows(n, nnz), A.lanes_per_row, row_ptr);
         A.v64 = dv;
         solve_result r;
         if (precision == NEON_PRECISION_FP64)
@@ -316,16 +363,20 @@ int neon_krylov_solve_csr_noalloc(neon_context* ctx, int solver, int criterion, 
         clear_flag_kernel<<<1, 64, 0, s>>>(flag);
         int const grid = int(std::min<int64_t>(1024, std::max<int64_t>(1, (std::max<int64_t>(nnz, n) + 255) / 256)));
         check_csr_kernel<<<grid, 256, 0, s>>>(n, nnz, row_ptr, col, flag);
+        int const lanes = lanes_for(double(nnz) / n);
+        csr_evenness_kernel<<<1, 256, 0, s>>>(n, nnz, ctx->engine->csr_block_rows(n, nnz), lanes, row_ptr, flag);
         NEON_CHECK_HIP(hipGetLastError());
-        if (ctx->engine->read_scalar(flag) != 0.0)
+        double const verdict = ctx->engine->read_scalar(flag);
+        if (verdict == 1.0)
             throw status_error(NEON_BAD_ARGUMENT, "malformed CSR arrays (row pointers or column indices)");
         linear_operator A;
         A.n = n;
         A.node_block = false;
         A.nnz = nnz;
+        A.uneven = verdict != 0.0;
         A.rp = row_ptr;
         A.ci = col;
-        A.lanes_per_row = lanes_for(double(nnz) / n);
+        A.lanes_per_row = lanes;
         A.v64 = val;
         double* minv = vec;
         krylov_work w;

@@ -111,7 +111,8 @@ struct sym_matrix; // krylov_kernels.hpp
 struct linear_operator
 {
     int64_t n = 0;
-    int64_t nnz = 0; // generic CSR layout only
+    int64_t nnz = 0;     // generic CSR layout only
+    bool uneven = false; // generic CSR layout: not for the resident grid (csr_grid_pays)
     bool node_block = false;
     // node-block layout
     int32_t nodes = 0;
@@ -260,6 +261,8 @@ public:
 
     hipStream_t stream() const { return s_; }
     int vec_blocks(int64_t n) const;
+    // rows of a workgroup of the resident grid for a CSR system
+    int64_t csr_block_rows(int64_t n, int64_t nnz) const;
     kernel_profiler* prof = nullptr;
     // iterations between convergence polls from the host
     int poll_every = 16;

@@ -621,8 +621,12 @@ struct grid_kept : grid_sliced<LAY>
 // add up each row's part of the chunk.  With lanes assigned to rows instead, as in
 // spmv_csr_kernel, the dependent loads of one row pointer, its columns and x are paid once per
 // four rows: 95 us against 37 us for the launch's 32 wavefronts per compute unit (7.6 M entries).
+// A row with more than kCsrLong entries in a chunk is added up by a wavefront (four lanes take 20 us for
+// a chunk of one row), in workgroups that have such rows: 20,000 rows, 64 of them full, 12.9 -> 1.3 ms
+// per iteration; workgroups without keep the loop without the list (with it 4 % slower at 1 M rows).
 constexpr int kCsrPerThread = 8;
-constexpr int kCsrChunk = kGridThreads * kCsrPerThread;
+constexpr int kCsrLong = 256;
+static_assert(kCsrChunk == kGridThreads * kCsrPerThread);
 template <typename VT>
 struct grid_csr
 {
@@ -667,10 +671,14 @@ struct grid_csr
             v[u] = on ? val[p] : VT(0);
         }
     }
+    bool any_long; // the block has rows of more than kCsrLong entries
     __device__ void hold(grid_shape const& g, const int32_t* ptr)
     {
         int const c = count(g);
         load(c > 0 ? ptr[0] : 0, c > 0 ? ptr[c] : 0);
+        int found = 0;
+        for (int q = threadIdx.x; q < c; q += kGridThreads) found |= ptr[q + 1] - ptr[q] > kCsrLong;
+        any_long = __syncthreads_or(found) != 0;
     }
     template <typename AT>
     __device__ AT result(grid_shape const&, const AT* y, const AT*, int lr) const
@@ -678,12 +686,13 @@ struct grid_csr
         return y[lr];
     }
     // a block of one chunk keeps it in registers; otherwise the last chunk's turn loads the first again
-    template <typename XT, typename AT, typename XV>
-    __device__ void product(grid_shape const& g, const int32_t* ptr, bool, XV x, AT* y, AT* part)
+    template <bool LONG, typename XT, typename AT, typename XV>
+    __device__ void chunks(grid_shape const& g, const int32_t* ptr, XV x, AT* y, AT* part)
     {
-        __shared__ int next_row;
+        __shared__ int next_row, longs, long_row[LONG ? kCsrChunk / kCsrLong : 1];
         int const c = count(g);
         int const tid = threadIdx.x;
+        if (LONG && tid == 0) longs = 0;
         for (int q = tid; q < c; q += kGridThreads) y[q] = AT(0);
         int64_t const beg = c > 0 ? ptr[0] : 0, end = c > 0 ? ptr[c] : 0;
         int ra = 0; // the chunk's first row
@@ -703,21 +712,49 @@ struct grid_csr
                 int64_t const lo = ptr[q], hi = ptr[q + 1];
                 if (lo >= c1) break;
                 int const a = int((lo > c0 ? lo : c0) - c0), b = int((hi < c1 ? hi : c1) - c0);
-                AT s = AT(0);
-                for (int p = a + sub; p < b; p += 4) s += part[p];
-                s += __shfl_xor(s, 1, 64);
-                s += __shfl_xor(s, 2, 64);
-                if (sub == 0)
+                if (LONG && b - a > kCsrLong)
                 {
-                    if (b > a) y[q] += s;
-                    // the one row that holds the chunk's last entry
-                    if (hi >= c1 && hi > lo) next_row = hi == c1 ? q + 1 : q;
+                    if (sub == 0) long_row[atomicAdd(&longs, 1)] = q;
                 }
+                else
+                {
+                    AT s = AT(0);
+                    for (int p = a + sub; p < b; p += 4) s += part[p];
+                    s += __shfl_xor(s, 1, 64);
+                    s += __shfl_xor(s, 2, 64);
+                    if (sub == 0 && b > a) y[q] += s;
+                }
+                // the one row that holds the chunk's last entry
+                if (sub == 0 && hi >= c1 && hi > lo) next_row = hi == c1 ? q + 1 : q;
             }
             __syncthreads();
             ra = next_row;
+            if constexpr (LONG)
+            {
+                int const lane = tid & 63, listed = longs;
+                for (int k = tid >> 6; k < listed; k += kGridWaves)
+                {
+                    int const q = long_row[k];
+                    int64_t const lo = ptr[q], hi = ptr[q + 1];
+                    int const a = int((lo > c0 ? lo : c0) - c0), b = int((hi < c1 ? hi : c1) - c0);
+                    AT s = AT(0);
+                    for (int p = a + lane; p < b; p += 64) s += part[p];
+                    s = wave_total(s);
+                    if (lane == 0) y[q] += s;
+                }
+                __syncthreads();
+                if (tid == 0) longs = 0;
+            }
         }
         __syncthreads();
+    }
+    template <typename XT, typename AT, typename XV>
+    __device__ void product(grid_shape const& g, const int32_t* ptr, bool, XV x, AT* y, AT* part)
+    {
+        if (any_long)
+            chunks<true, XT, AT>(g, ptr, x, y, part);
+        else
+            chunks<false, XT, AT>(g, ptr, x, y, part);
     }
 };
 

@@ -163,11 +163,16 @@ bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_
 // Shape of a CSR grid: at least 64 rows per block.  A system of at most two chunks of entries takes
 // one block, whose exchanges stay within the workgroup and which gathers p from LDS (210 rows, 3,952
 // entries: 3.4 us per iteration against 5.6 with four blocks).
-bool shape_csr(grid_shape& g, int64_t n, int64_t nnz, int units, vector_need need)
+int64_t csr_rows(int64_t n, int64_t nnz, int units)
 {
     int64_t const most = std::min(units, kGridMaxBlocks);
-    int64_t rows = nnz <= 2 * kCsrChunk && n <= 2 * kGridThreads ? n : std::max<int64_t>(64, (n + most - 1) / most);
-    rows = (rows + 15) / 16 * 16;
+    int64_t const rows = nnz <= 2 * kCsrChunk && n <= 2 * kGridThreads ? n : std::max<int64_t>(64, (n + most - 1) / most);
+    return (rows + 15) / 16 * 16;
+}
+
+bool shape_csr(grid_shape& g, int64_t n, int64_t nnz, int units, vector_need need)
+{
+    int64_t const rows = csr_rows(n, nnz, units);
     if (rows > 64 * kGridThreads) return false;
     g.n = n;
     g.rows = int32_t(rows);
@@ -201,9 +206,11 @@ bool shape_of(grid_shape& g, linear_operator const& A, int units, vector_need ne
         return shape_sliced(g, A.n, A.sym_slots / 8, 1.0 + A.sym_mean, 1 + A.sym_entries, units, need);
     if (A.node_block && A.sell)
         return shape_sliced(g, A.n, (A.slices + 7) / 8, A.sell_mean, A.sell_steps, units, need);
-    return !A.node_block && shape_csr(g, A.n, A.nnz, units, need);
+    return !A.node_block && !A.uneven && shape_csr(g, A.n, A.nnz, units, need);
 }
 } // namespace
+
+int64_t krylov_engine::csr_block_rows(int64_t n, int64_t nnz) const { return csr_rows(n, nnz, std::max(grid_units_, 1)); }
 
 // What the resident grids need beyond a solve's own vectors: with the engine, so that a solve in
 // vectors of the caller's allocates nothing
@@ -383,7 +390,7 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
             done = with(grid_sliced<lay>{l});
     }
     else
-        done = with(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}});
+        done = with(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}, false});
     if (!done) return false;
     out = finish_solve(*host_state_, criterion);
     out.spmv = out.iterations + (criterion == NEON_STOP_RELATIVE && host_state_->done == KRYLOV_CONVERGED ? 1 : 0);
@@ -446,7 +453,7 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
             done = launch(grid_sliced<lay>{l});
     }
     else
-        done = launch(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}});
+        done = launch(grid_csr<double>{csr_matrix{int32_t(n), A.rp, A.ci}, A.v64, {}, {}, false});
     if (!done) return false;
     out = finish_bicg(*host_state_, criterion);
     return true;

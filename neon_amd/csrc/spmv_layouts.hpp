@@ -58,6 +58,19 @@ struct csr_matrix
     const int32_t* ci;
 };
 
+// Entries that a workgroup of the resident CSR grid takes at a time.  Its workgroups own equal runs of
+// rows, so the one with the most entries sets the pace: 4 to 7 us for each chunk that it has more than
+// the mean, against what the launches lose on the exchanges and passes (10 us, 2 us per mean chunk) and
+// on the longest row, which they give `lanes` lanes (some 0.25 us per step).  Per iteration, grid /
+// launches before this rule: 100,000 rows of 7 entries and 400 more rows of 20, 60, 160, 500 entries side by side
+// 19 / 29, 32 / 35, 77 / 47, 223 / 82 us; 64 of 2,000 133 / 126; 4 of 5,000 31 / 129; one of 16,457 29 / 352.
+constexpr int kCsrChunk = 4096;
+__host__ __device__ inline bool csr_grid_pays(int64_t largest_block, double mean_block, int64_t longest_row, int lanes)
+{
+    return 5.0 * (double(largest_block) - mean_block) / kCsrChunk
+           <= 10.0 + 2.0 * mean_block / kCsrChunk + 0.25 * double(longest_row) / lanes;
+}
+
 // Sliced node-block layout: a copy of the node-block values in which every wavefront load
 // reads one contiguous span.  Slice s holds the 64 consecutive nodes 64 s ... 64 s + 63 (lane l:
 // node snode[64 s + l]; an empty lane past the last node, snode -1 - m, gathers like node m and

@@ -135,6 +135,61 @@ def test_cg_on_host_csr(ctx, n, per_row, long_rows):
     _check(A, b, grid, launches)
 
 
+def _with_rows(n, lengths, seed):
+    """Diagonally dominant, symmetric: the first rows have these lengths (diagonal included), over the
+    columns after theirs; the others the diagonal, their parts of those and a neighbour."""
+    rng = np.random.default_rng(seed)
+    i = np.concatenate([np.full(k - 1, r) for r, k in enumerate(lengths)])
+    m = len(lengths)
+    j = np.concatenate([np.sort(rng.choice(np.arange(m, n), k - 1, replace=False)) for k in lengths])
+    far = np.arange(m, n - 1)
+    i, j = np.concatenate([i, far]), np.concatenate([j, far + 1])
+    S = sp.coo_matrix((rng.uniform(-1, 1, len(i)), (i, j)), shape=(n, n)).tocsr()
+    S = S + S.T
+    S = (S + sp.diags(np.abs(S).sum(axis=1).A1 * 1.05 + 1.0)).tocsr()
+    S.sort_indices()
+    assert list(np.diff(S.indptr)[:m]) == list(lengths)
+    return S, rng.standard_normal(n)
+
+
+# Rows at the length from which a wavefront adds them up (256 entries of a chunk), in one workgroup and
+# in several; a chunk full of such rows; rows of a chunk and more; and rows so unequal that the launch
+# loop takes the system
+@pytest.mark.parametrize("n,lengths", [(600, [255, 256, 257, 258]), (5000, [255, 256, 257, 258, 512]),
+                                       (5000, [257] * 40), (40000, [4095, 4096, 4097, 9000]), (70000, [300] * 64),
+                                       (30000, [20000] * 64)])
+def test_cg_and_bicgstab_on_long_rows(ctx, n, lengths):
+    print(n, len(lengths), flush=True)
+    A, b = _with_rows(n, lengths, n)
+    for cls in (neon_amd.conjugate_gradient_hip, neon_amd.biconjugate_gradient_stabilised_hip):
+        grid, launches = _both(ctx, lambda: _solve_csr(ctx, cls, A, b))
+        for x, its, _ in (grid, launches):
+            assert np.linalg.norm(b - A @ x) <= 2e-10 * np.linalg.norm(b)
+        assert abs(grid[1] - launches[1]) <= 3 + 0.15 * launches[1], (grid[1], launches[1])
+
+
+def test_unequal_rows_cost_no_more_than_the_launch_loop(ctx):
+    """64 full rows of 20,000: the solve must not be far slower than the launch loop (it was 13 times).
+    The least of three calls each; 2 for the scatter (the launch loop's calls are timed per kernel)."""
+    import time
+
+    A, b = _with_rows(20064, [20000] * 64, 3)
+    arrays = (A.indptr, A.indices, A.data)
+
+    def timed():
+        times = []
+        for _ in range(3):
+            start = time.perf_counter()
+            _solve_csr(ctx, neon_amd.conjugate_gradient_hip, arrays, b)
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    timed()
+    grid, launches = _both(ctx, timed)
+    print(grid, launches, flush=True)
+    assert grid <= 2.0 * launches
+
+
 def _chain(n, shift):
     return sp.diags([-np.ones(n - 1), np.full(n, 2.0 + shift), -np.ones(n - 1)], [-1, 0, 1], format="csr")
 
