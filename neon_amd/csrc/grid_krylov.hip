@@ -144,9 +144,15 @@ bool shape_sliced(grid_shape& g, int64_t n, int32_t per_xcd, double mean, int32_
         t.rounds = (per_xcd + groups * most - 1) / (groups * most);
         if (wps == 4 && t.rounds > 1) continue;
         // from four rounds on the launches' own dispatch spreads the slices better and the grid's
-        // exchanges no longer outweigh that: 1,073,733 dofs 97.3 us per iteration against 107.9 by
-        // launches, 1,215,672 dofs 130.8 against 123.0
+        // exchanges no longer outweigh that: 1,073,733 dofs 96.6 us per iteration against 105.1 by
+        // launches, 1,215,672 dofs 130.8 against 123.0; at three rounds if they are not full or their
+        // slices unequal (the items that every wavefront waits for against those there are): 815,409
+        // dofs 82.0 against 79.6, long bars on the full copy 960,048 dofs 135 against 126, 1,026,027 dofs
+        // 150 against 120; full ones on the full copy 1,029,000 dofs 151 against 157
         if (t.rounds > 3 && wps == 1) continue;
+        if (t.rounds == 3 && wps == 1
+            && t.rounds * (2.0 + most_items) > 1.4 * (2.0 + mean) * per_xcd / (groups * most))
+            continue;
         t.per_xcd = std::min(most, (per_xcd + groups - 1) / groups);
         t.blocks = 8 * t.per_xcd;
         t.rows = t.rounds * groups * 192;
