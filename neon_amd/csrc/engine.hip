@@ -634,7 +634,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
     // arithmetic; x64 stays unscaled (the folds scale the steps back) and the FP64 residuals
     // r = b - K x64 use A, the unscaled FP32 values, so convergence is judged on K as without it
     bool const scaled = minv64_scaled != nullptr;
-    linear_operator Ak = scaled ? *scaled_op : A; // its products alternate in order
+    linear_operator Ak = scaled ? *scaled_op : A; // its products on a symmetric copy alternate in order
     // the iterations without a decision with their vector part in one launch (scaled system), and all
     // again without if that gave up
     int64_t launched = 0;
@@ -659,7 +659,7 @@ solve_result krylov_engine::cg_mixed_run(const linear_operator& A, const double*
                 krylov_state* cur = st + (launched & 1);
                 krylov_state* nxt = st + ((launched + 1) & 1);
                 int const tok = prof ? prof->begin(s_, NEON_KERNEL_SPMV_FP32) : -1;
-                Ak.back = int(launched & 1);
+                Ak.back = Ak.sym ? int(launched & 1) : 0;
                 Ak.apply32(s_, p32, Ap32, part_pAp, cur);
                 if (prof) prof->end(s_, tok);
                 // the reliable-update / true-residual convergence test runs every refine_every

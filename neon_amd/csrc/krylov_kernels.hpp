@@ -156,10 +156,10 @@ __global__ __launch_bounds__(kBlock) void spmv_nb_kernel(nb_matrix A, const VT* 
 // NT: the values are read with nontemporal loads (streamed past the caches, which keep x).
 // back: the slices in the opposite order.  A solver alternates it from product to product, so that a
 // product starts with the part of the matrix that the one before read last and the 256 MB
-// memory-side cache may still hold: 91^3 nodes, mixed precision 1,534 -> 1,397 ms per load step
-// (147 -> 134 us per iteration), 80^3 FP64 384 -> 355 ms per solve.  Whole groups of 32 change places,
-// so that a slice stays on its XCD, whose L2 may hold it: 20^3, 28^3, 30^3 cells numbered by a mesh
-// generator, mixed, 90.5, 138.2, 154.2 ms with the XCD changing, 86.0, 133.1, 148.5 here.
+// memory-side cache may still hold: per iteration, one order against alternating, symmetric copy FP32 96^3
+// cells 140 -> 126 us, FP64 80^3 169 -> 158, 96^3 279 -> 266; full copy FP64 96^3 388 -> 383, 70^3 164.5 -> 162.5
+// (FP32 none, 70^3 104 -> 107.5: the mixed solver alternates on the symmetric copy only).  Whole groups of
+// 32 change places, so that a slice stays on its XCD, whose L2 may hold it.
 template <bool I16, bool NT, typename VT, typename XT, typename YT, typename AT, bool DOT, int MODE>
 __global__ __launch_bounds__(256) void spmv_sell_kernel(sell_matrix A, const VT* __restrict__ val,
                                                         const XT* __restrict__ x, YT* __restrict__ y,
