@@ -102,24 +102,47 @@ def test_newton_cube_parity(ctx, n, top):
     assert (dr["damage"] > 0).all()
 
 
-@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (3, 3, 1), (3, 3, 3)])
-def test_return_map_groups_parity(ctx, dims):
-    """The return map handles 64 yielding points per workgroup, taken from a list: one element (8
-    points), exactly one group, one point group more, and several, some of the points elastic (the
-    pull grows from nothing along x), against the oracle (tolerances of the sequence test)."""
-    print(dims, flush=True)
+def _update_both(ctx, dims, displacement):
+    """One update from rest on the device and in the oracle; the oracle's state, held to the
+    device's with the tolerances of the sequence test."""
     X, conn, _ = problems.box_mesh(*dims, L=(1.0, 1.0, 1.0), jitter=0.1)
     params = np.repeat(problems.damage_cube(1).params[:1], len(conn), axis=0)
     mg = neon_amd.DeviceMesh(X, conn, params, model=neon_amd.MODEL_J2_DAMAGE, context=ctx, damage=CONST)
     mr = orc.Model(X, conn, params, model=orc.MODEL_J2_DAMAGE)
     mr.set_damage(CONST)
-    u = np.zeros_like(X)
-    u[:, 2] = 0.0025 * X[:, 2] * X[:, 0]
-    u[:, 0] = -0.0007 * X[:, 0] * X[:, 2]
-    u = u.reshape(-1)
+    u = displacement(X).reshape(-1)
     mg.set_displacement(u)
     mg.update_internal_variables(1e-3)
     assert mr.update(u, 1e-3) == orc.OK
     sg, sr = mg.qp_state(), mr.qp_state()
     for key in ("sigma", "D", "eps_p", "ebar", "vm"):
         _close(sg[key], sr[key], 1e-9, key)
+    return sr
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (3, 3, 1), (3, 3, 3)])
+def test_return_map_groups_parity(ctx, dims):
+    """The return map handles 64 yielding points per workgroup, taken from a list.  Here the pull grows
+    from nothing along x, so that some of the points stay elastic and the list skips them: less than
+    a group, around one group, and several, against the oracle."""
+    print(dims, flush=True)
+
+    def displacement(X):
+        u = np.zeros_like(X)
+        u[:, 2] = 0.0025 * X[:, 2] * X[:, 0]
+        u[:, 0] = -0.0007 * X[:, 0] * X[:, 2]
+        return u
+
+    state = _update_both(ctx, dims, displacement)
+    flowed = int((state["ebar"] > 0).sum())
+    assert 0 < flowed < state["ebar"].size, flowed
+
+
+# one element; exactly one group, and two; a group and eight points; and more points (39,304) than the
+# launch's 512 workgroups take at once, so that some take a second group
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 2, 2), (4, 2, 2), (3, 3, 1), (17, 17, 17)])
+def test_return_map_full_groups_parity(ctx, dims):
+    """Every point yields (a uniform pull well past the yield stress), against the oracle."""
+    print(dims, flush=True)
+    state = _update_both(ctx, dims, lambda X: 0.0025 * X * [-0.3, -0.3, 1.0])
+    assert (state["ebar"] > 0).all() and state["ebar"].size == 8 * np.prod(dims)
