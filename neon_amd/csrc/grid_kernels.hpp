@@ -55,7 +55,7 @@ struct grid_shape
     int32_t blocks = 0;    // of the grid
     int32_t per_xcd = 0;   // blocks per XCD
     int32_t rounds = 0;    // sliced layouts
-    int32_t wps = 1;       // wavefronts per slice: 1, 2, 4 or 8
+    int32_t wps = 1;       // wavefronts per slice: 1, 4 or 8
     int32_t rows = 0;      // rows of a block (capacity)
     bool all = false;      // every vector of the recurrence in LDS
     int64_t lds = 0;       // bytes of dynamic LDS
@@ -91,10 +91,6 @@ __device__ inline int here(int tid)
 }
 
 __device__ inline void publish(double* p, double v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void publish(float* p, float v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -567,7 +563,6 @@ struct grid_sliced
         switch (g.wps)
         {
         case 1: product_shared<1, XT, AT>(g, first_row, back, x, y, part); break;
-        case 2: product_shared<2, XT, AT>(g, first_row, back, x, y, part); break;
         case 4: product_shared<4, XT, AT>(g, first_row, back, x, y, part); break;
         default: product_shared<8, XT, AT>(g, first_row, back, x, y, part); break;
         }
