@@ -119,7 +119,9 @@ int neon_context_synchronize(neon_context* ctx);
  * whose timing is std::chrono prints) ----
  * While enabled, every SpMV launch of the Krylov solvers and every assembly call is
  * bracketed by events; counts and summed milliseconds accumulate per kernel class until
- * read with reset.  Classes: */
+ * read with reset.  A timed solve always takes the launch loop: systems that otherwise run whole
+ * batches of iterations in one launch (CG up to about 1 M dofs, BiCGSTAB up to 0.4 M) then take
+ * longer, and their last bits differ (the sums' order).  Classes: */
 #define NEON_KERNEL_SPMV_FP64 0     /* node-block SpMV, FP64 values/vectors */
 #define NEON_KERNEL_SPMV_FP32 1     /* node-block SpMV, FP32 values/vectors (mixed inner) */
 #define NEON_KERNEL_RESIDUAL_FP64 2 /* b - K x in FP64 (mixed reliable updates) */
@@ -132,7 +134,9 @@ int neon_context_profile_read(neon_context* ctx, int kernel_class, int reset, in
  * A is square, row-major CSR, int32 indices, FP64 values.  x is overwritten.  With
  * precision NEON_PRECISION_MIXED the inner iterations run in FP32 with FP64 reliable
  * updates of b - A x (only NEON_SOLVER_CG).  iterations / error receive the solver's
- * iteration count and final residual measure in the stopping rule's own form. */
+ * iteration count and final residual measure in the stopping rule's own form.  The context keeps
+ * the call's device memory for the next one, up to 256 MiB (larger blocks are freed at the call's
+ * end). */
 int neon_krylov_solve_csr(neon_context* ctx, int solver, int criterion, int precision, int32_t n, int64_t nnz,
                           const int32_t* row_ptr, const int32_t* col, const double* val, const double* b,
                           double* x, double tolerance, int32_t max_iterations, int32_t* iterations,

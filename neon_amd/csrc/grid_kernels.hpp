@@ -22,10 +22,11 @@
 // fill whole 128-byte lines of p, so no line is written by two workgroups.
 //
 // Progress.  The grid has at most one workgroup per compute unit and the host holds that many
-// compute units for it against the other grids of the process, so all workgroups run at once
-// as soon as ordinary kernels have left room.  Should another process keep some of them out, the
-// waiting ones give up after a bounded time, raise the abort word and return; every workgroup
-// checks that word when it starts, and the host then solves with the launch-per-phase loop.
+// compute units for it against the other grids of the process (batch by batch where another solve
+// waits for some), so all workgroups run at once as soon as ordinary kernels have left room.  Should
+// another process keep some of them out, the waiting ones give up after a bounded time, raise the
+// abort word and return; every workgroup checks that word when it starts, and the host then solves
+// with the launch-per-phase loop, as it does the context's next solves for a while.
 #pragma once
 
 #include "spmv_layouts.hpp"
@@ -759,7 +760,7 @@ struct grid_csr
 // With b the launch starts the solve (x = 0, r = b, p = M^-1 r), else it continues the one in
 // *st.  Ring buffer k holds the p of the launch's iteration k; x, r and p leave through global
 // memory (p in buffer 0).  A p's place in LDS takes z = M^-1 r once A p is used.  ALL: x and M^-1
-// are in LDS too; else they are read from global memory ahead of the exchange that waits for p.Ap.
+// are in LDS too; else they are read from global memory before the exchange of p.Ap, which waits for them.
 // A thread handles the local rows tid, tid + kGridThreads, ... (at most kGridElems).
 template <bool ALL>
 constexpr int kGridElems = ALL ? 8 : 12;
@@ -1249,9 +1250,11 @@ __global__ __launch_bounds__(kGridThreads) void bicg_grid_kernel(ROWS rows, grid
 // The scalars and vectors of one iteration between two products of the launch loops, in one launch
 // in place of three (totals, r update, x and p update): the total of p.Ap from the product's partials,
 // r -= alpha A p with r.z (and r.r), the exchange of those sums, and x += alpha p, p = z + beta p.  r
-// stays in registers between the two halves, x and p are requested ahead of the exchange: 7 vector
-// passes instead of 8 (FP32 on the Jacobi-scaled copy, z = r), 8 instead of 10 (FP64).  One workgroup
-// per compute unit; a thread's elements past its kVectorKeep groups are read again.  DECIDE: the scalar rules of the loop, s <- the next state, returns beta.
+// stays in registers between the two halves, as do x and p (read before the exchange, which waits for
+// them: 31 us at 1.6 M dofs, 102 MB that a copy moves in 17): 7 vector passes instead of 8 (FP32 on the
+// Jacobi-scaled copy, z = r), 8 instead of 10 (FP64).  One workgroup per compute unit; a thread's
+// elements past its kVectorKeep groups are read again.  DECIDE: the scalar rules of the loop, s <- the
+// next state, returns beta.
 constexpr int kVectorThreads = 1024;
 constexpr int kVectorKeep = 3; // 16-byte groups of each vector that a thread keeps
 
