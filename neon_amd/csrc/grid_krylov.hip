@@ -186,11 +186,12 @@ bool shape_csr(grid_shape& g, int64_t n, int64_t nnz, int units, vector_need nee
     return fit_lds(g, kCsrChunk * 8 + 4 * (rows + 1), need);
 }
 
+// Every solve sets the same limit: another thread may launch the kernel with more LDS than this one needs
 template <typename K>
-void allow_lds(K kernel, int64_t bytes)
+void allow_lds(K kernel)
 {
     NEON_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       int(bytes)));
+                                       int(kGridLds)));
 }
 
 sym_matrix sym_of(linear_operator const& A)
@@ -356,7 +357,7 @@ bool krylov_engine::cg64_grid(const linear_operator& A, const double* b, double*
     krylov_state* st = state_.data() + 2;
     unit_hold hold(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto kernel, auto rows) {
-        allow_lds(kernel, g.lds);
+        allow_lds(kernel);
         return grid_run(hold, [&, kernel](bool first) {
             kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, first ? b : nullptr, x, r, minv,
                                                                   st, grid_next(uint32_t(3 * iters + 2)), iters,
@@ -436,7 +437,7 @@ bool krylov_engine::bicgstab64_grid(const linear_operator& A, const double* b, d
     unit_hold hold(grid_device_, g.blocks, grid_units_);
     auto launch = [&](auto rows) {
         auto kernel = bicg_grid_kernel<decltype(rows)>;
-        allow_lds(kernel, g.lds);
+        allow_lds(kernel);
         return grid_run(hold, [&, kernel](bool first) {
             kernel<<<g.blocks, kGridThreads, size_t(g.lds), s_>>>(rows, g, ring, stride, b, x, r, r0, p, v, minv, st,
                                                                   grid_next(uint32_t(7 * iters + 1)), first ? 1 : 0,

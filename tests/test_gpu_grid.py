@@ -467,6 +467,33 @@ def test_two_contexts_share_the_gpu():
         assert np.array_equal(results[k][0], results[k][1]) and np.array_equal(results[k][0], results[k][2])
 
 
+def test_threads_launch_one_kernel_with_different_lds():
+    """Two threads whose solves take the same kernel, one with 44 KB of LDS per workgroup and one with
+    95 KB: each solve gets what it needs whatever the other asked for last."""
+    import threading
+
+    systems = [_spd(70001, 8, 50), _spd(400000, 4, 51)]
+    results = {0: [], 1: []}
+
+    def work(k):
+        c = neon_amd.Context(0)
+        try:
+            for _ in range(12):
+                results[k].append(_solve_csr(c, neon_amd.conjugate_gradient_hip, *systems[k])[0])
+        finally:
+            c.close()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in results]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k, (A, b) in enumerate(systems):
+        assert len(results[k]) == 12
+        assert np.linalg.norm(b - A @ results[k][0]) <= 1.1e-10 * np.linalg.norm(b)
+        assert all(np.array_equal(x, results[k][0]) for x in results[k])
+
+
 # a large solve in the launch loop with its one-launch vector part (mixed, FP64) and in the resident grid,
 # each a good part of a second long (none reaches its tolerance)
 @pytest.mark.parametrize("dims,precision,tol,limit", [((104, 102, 101), "mixed", 1e-30, 6000),
