@@ -213,12 +213,20 @@ class unit_pool;
 class unit_hold
 {
 public:
-    unit_hold(int device, int count, int units);
+    unit_hold(int device, int blocks, int units);
     ~unit_hold();
     unit_hold(unit_hold const&) = delete;
     unit_hold& operator=(unit_hold const&) = delete;
     bool wanted() const;
     void yield();
+    // compute units held for `blocks` workgroups on a GPU of `units`: workgroups go to the 8 XCDs in turn,
+    // whatever room these have, so counts are taken in whole turns; otherwise grids that fit by their
+    // sum (250 and 6 workgroups, say) overfill an XCD, and each may wait for a compute unit the other has
+    static constexpr int held(int blocks, int units)
+    {
+        int const whole = (blocks + 7) / 8 * 8;
+        return whole <= units ? whole : units;
+    }
 
 private:
     unit_pool& pool_;

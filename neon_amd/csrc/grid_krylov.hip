@@ -86,7 +86,8 @@ private:
     std::atomic<uint64_t> arrived_{0}, served_{0};
 };
 
-unit_hold::unit_hold(int device, int count, int units) : pool_(unit_pool::of(device)), count_(count), units_(units)
+unit_hold::unit_hold(int device, int blocks, int units)
+    : pool_(unit_pool::of(device)), count_(held(blocks, units)), units_(units)
 {
     pool_.take(count_, units_);
 }

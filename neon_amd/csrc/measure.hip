@@ -309,4 +309,7 @@ int neon_test_grid_epoch(neon_context* ctx, uint32_t epoch)
     });
 }
 
+// The compute units that a resident grid of `blocks` workgroups holds on a GPU of `units` (for its test).
+int neon_test_units_held(int blocks, int units) { return unit_hold::held(blocks, units); }
+
 } // extern "C"

@@ -1,6 +1,7 @@
 """CPU checks of the C ABI library: it loads, exports every function that
 include/neon_hip.h declares, and its host-only parts (mesh generator, random streams,
 argument checks) behave.  No compute call needs a GPU here."""
+import ctypes as C
 import pathlib
 import re
 
@@ -38,6 +39,29 @@ def test_probes_live_in_the_measurement_library_only():
     assert set(names) == set(_capi.MEASURE_SIGNATURES)
     product = _capi.lib()
     assert not any(hasattr(product, n) for n in names)
+
+
+def test_resident_grids_that_the_pool_admits_together_fit_every_xcd():
+    """Workgroup i of a grid runs on XCD i % 8.  Any grids whose held units add up to at most the GPU's
+    (256, 32 per XCD) have room on each XCD at once, and a grid never asks for more than there are."""
+    held = _capi.measure_lib().neon_test_units_held
+    held.restype, held.argtypes = C.c_int, [C.c_int, C.c_int]
+
+    def load(blocks):
+        return np.bincount(np.arange(blocks) % 8, minlength=8)
+
+    rng = np.random.default_rng(0)
+    for _ in range(2000):
+        free, total = 256, np.zeros(8, int)
+        while True:
+            blocks = int(rng.integers(1, 257))
+            if held(blocks, 256) > free:
+                break
+            free -= held(blocks, 256)
+            total += load(blocks)
+        assert (total <= 32).all()
+    for units in (1, 3, 8, 32, 100, 256):
+        assert all(b <= held(b, units) <= units for b in range(1, units + 1))
 
 
 def test_no_device_is_a_loud_error_here():
